@@ -15,7 +15,8 @@
 // (batch 64) took 12 us, latency-bound on 14 chunks per wavefront.
 //
 // Activations are either fp32 (W8A32: DequantizeLinear(W) -> Gemm with
-// unquantised inputs) or E4M3 (W8A8, decoded per chunk).
+// unquantised inputs, where few rows and panels make the matrix-core kernel's
+// barriers the cost: gemm_w8a32.hip) or E4M3 (W8A8, decoded per chunk).
 #include "lcml_internal.hpp"
 
 namespace lcml {

@@ -1,0 +1,83 @@
+"""W8A32 on the bf16 matrix cores: fp32 activations in three exact pieces.
+
+Against a 64-bit product with a bound of fp32 sums: the pieces' products are
+exact and a sum of K of them in any order is within K * 2^-24 * sum|a b| of
+the exact one (the scale, bias and output rounding add three more)."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from luisaml_amd import capi, synth
+
+pytestmark = pytest.mark.gpu
+
+
+def run(dev, a, qw, sw, bias, pad=0, shift=0, out_dtype=torch.float32):
+    M, K = a.shape
+    buf = torch.zeros(shift + M * (K + pad), dtype=torch.float32, device=dev)
+    va = buf[shift:].view(M, K + pad)[:, :K]
+    va.copy_(torch.from_numpy(a))
+    bp = capi.pack_weight(torch.from_numpy(qw).to(dev), True)
+    return capi.gemm_w8a32(va, bp, torch.from_numpy(sw).to(dev), qw.shape[0], K, c=torch.from_numpy(bias).to(dev),
+                           out_dtype=out_dtype)
+
+
+def weights(N, K, seed):
+    w = synth.normal(seed, (N, K), std=0.05)
+    sw = oracle.channel_scales(w, axis=0)
+    return oracle.quantize(w, sw, axis=0), sw
+
+
+def check(y, a, qw, sw, bias):
+    K = a.shape[1]
+    B = oracle.e4m3_to_float(qw).astype(np.float64) * sw.astype(np.float64)[:, None]
+    ref = a.astype(np.float64) @ B.T + bias
+    bound = (K + 3) * 2.0 ** -24 * (np.abs(a).astype(np.float64) @ np.abs(B).T + np.abs(bias))
+    assert np.all(np.abs(y.astype(np.float64) - ref) <= bound)
+
+
+# 16x1, 16x2 and 32x3 tiles with row, column and K remainders (K at the edges
+# of a 16-k chunk, a 64-k step, a 128-k block and the parts), and the
+# vector-ALU kernel's sizes
+@pytest.mark.parametrize("M,N,K", [(1, 64, 100), (17, 4100, 1000), (65, 1030, 65), (33, 11000, 127), (40, 11008, 129),
+                                   (129, 6000, 200), (100, 11007, 64), (127, 8200, 1), (96, 12300, 528)])
+@pytest.mark.parametrize("pad,shift", [(0, 0), (4, 4), (3, 1)])
+def test_w8a32_against_64_bits(dev, M, N, K, pad, shift):
+    a = synth.normal(M, (M, K)) * np.exp(synth.normal(M + 1, (M, K), std=3.0)).astype(np.float32)
+    qw, sw = weights(N, K, N)
+    bias = synth.normal(3, (N,), std=0.01)
+    check(run(dev, a, qw, sw, bias, pad, shift).cpu().numpy(), a, qw, sw, bias)
+
+
+@pytest.mark.parametrize("scale", [1e-38, 1e-30, 1e30])
+def test_w8a32_ends_of_the_range(dev, scale):
+    """Subnormal pieces, and values near the largest: the bound plus what the
+    smallest bf16 value (2^-133) drops of each activation."""
+    M, N, K = 40, 2048, 256
+    a = (synth.normal(1, (M, K)) * scale).astype(np.float32)
+    qw, sw = weights(N, K, 2)
+    sw = np.ones_like(sw)
+    B = oracle.e4m3_to_float(qw).astype(np.float64)
+    y = run(dev, a, qw, sw, np.zeros(N, np.float32)).cpu().numpy().astype(np.float64)
+    ref = a.astype(np.float64) @ B.T
+    bound = (K + 3) * 2.0 ** -24 * (np.abs(a).astype(np.float64) @ np.abs(B).T) + 2.0 ** -133 * np.abs(B).sum(1)
+    assert np.all(np.abs(y - ref) <= bound)
+
+
+@pytest.mark.parametrize("M,N", [(40, 2048), (40, 11008), (128, 11008)])
+def test_w8a32_infinities_and_nan(dev, M, N):
+    """inf and NaN activations (a NaN whose upper half is an infinity's among
+    them) give what the oracle's fma chain gives, in their own rows only."""
+    K = 130
+    a = synth.normal(5, (M, K))
+    a[3, 7], a[20, 129], a[21, 1] = np.inf, -np.inf, np.array(0x7F800001, np.uint32).view(np.float32)
+    a[22, 4], a[22, 5] = np.inf, -np.inf
+    qw, sw = weights(N, K, 6)
+    bias = np.zeros(N, np.float32)
+    y = run(dev, a, qw, sw, bias).cpu().numpy()
+    ref = oracle.gemm(a, oracle.dequantize(qw, sw, axis=0), transB=1)
+    assert np.array_equal(np.isnan(y), np.isnan(ref)) and np.array_equal(np.isinf(y), np.isinf(ref))
+    assert np.array_equal(np.sign(y[np.isinf(y)]), np.sign(ref[np.isinf(ref)]))
+    fin = np.isfinite(ref).all(1)
+    check(y[fin], a[fin], qw, sw, bias)
