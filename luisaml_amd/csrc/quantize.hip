@@ -21,26 +21,31 @@ typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 __device__ inline uint32_t enc4(f4 v, const Recip &d) { return quantize4(v.x, v.y, v.z, v.w, d); }
 
 
-// Vector path, per-tensor or per-axis with inner % 4 == 0 (one scale per
-// float4); requires x 16-byte and y 4-byte aligned.  Each thread encodes kU
+// one element by the plain definition
+__device__ inline void quantize_tail(const float *x, uint8_t *y, int64_t i, float s) {
+    y[i] = (uint8_t)e4m3_encode(__fdiv_rn(x[i], s));
+}
+
+// Vector path, per-tensor; requires x 16-byte and y 4-byte aligned.  Each thread encodes kU
 // float4s per pass, taken kThreads apart so that every load instruction of a
 // wavefront reads 1 KB and every store writes 256 contiguous bytes (kU = 4
 // measured a little faster than 8 or 16 on 16M-45M element tensors).  The first pass's loads are issued before
 // the scale is known (with a dynamic scale, its reduction from the partial
 // maxima overlaps them) and each later pass's before the previous pass's
-// stores.
+// stores.  The last n % 4 elements fall to the first threads (a launch of
+// their own cost 2-4 us).
 constexpr int kU = 4;
 
 template <bool FROM_AMAX>
 __global__ __launch_bounds__(kThreads) void k_quantize_vec(const float *__restrict__ x,
-                                                           uint8_t *__restrict__ y, int64_t n4,
-                                                           int64_t axis_len, int64_t inner,
+                                                           uint8_t *__restrict__ y, int64_t n,
                                                            const float *__restrict__ scale,
                                                            const uint32_t *__restrict__ part, int npart,
                                                            float *__restrict__ scale_out) {
     __shared__ float red[kThreads / 64];
     const f4 *x4 = reinterpret_cast<const f4 *>(x);
     uint32_t *y4 = reinterpret_cast<uint32_t *>(y);
+    const int64_t n4 = n >> 2;
     const int64_t stride = (int64_t)gridDim.x * kThreads * kU;
     int64_t i0 = (int64_t)blockIdx.x * kThreads * kU + threadIdx.x;
     f4 v[kU];
@@ -52,28 +57,21 @@ __global__ __launch_bounds__(kThreads) void k_quantize_vec(const float *__restri
         }
     };
     load(i0);
-    float s_tensor = 1.0f;
+    float s_tensor;
     if (FROM_AMAX) {
         s_tensor = scale_from_partials<kThreads>(part, npart, red);
         if (scale_out && blockIdx.x == 0 && threadIdx.x == 0) *scale_out = s_tensor;
-    } else if (axis_len == 1) {
+    } else {
         s_tensor = scale[0];
     }
     const Recip d_tensor = make_recip(s_tensor);
-    // per-tensor: the scale's range test is uniform, one branch outside the
-    // loop; per-axis: a scale (and its test) per float4
-    auto run = [&](auto mode) {
-        constexpr int MODE = decltype(mode)::value;  // 0: per-axis, 1: tensor fast, 2: tensor IEEE
+    // the scale's range test is uniform: one branch outside the loop
+    auto run = [&](auto fast) {
         for (; i0 < n4; i0 += stride) {
             uint32_t code[kU];
 #pragma unroll
-            for (int u = 0; u < kU; ++u) {
-                const int64_t i = i0 + (int64_t)u * kThreads;
-                if constexpr (MODE == 0)
-                    code[u] = enc4(v[u], make_recip(scale[((i * 4) / inner) % axis_len]));
-                else
-                    code[u] = quantize4_t<MODE == 1>(v[u].x, v[u].y, v[u].z, v[u].w, d_tensor);
-            }
+            for (int u = 0; u < kU; ++u)
+                code[u] = quantize4_t<decltype(fast)::value>(v[u].x, v[u].y, v[u].z, v[u].w, d_tensor);
             if (i0 + stride < n4) load(i0 + stride);
 #pragma unroll
             for (int u = 0; u < kU; ++u) {
@@ -82,19 +80,120 @@ __global__ __launch_bounds__(kThreads) void k_quantize_vec(const float *__restri
             }
         }
     };
-    if (!FROM_AMAX && axis_len != 1)
-        run(std::integral_constant<int, 0>{});
-    else if (d_tensor.fast)
-        run(std::integral_constant<int, 1>{});
+    if (d_tensor.fast)
+        run(std::true_type{});
     else
-        run(std::integral_constant<int, 2>{});
+        run(std::false_type{});
+    if (blockIdx.x == 0 && threadIdx.x < (n & 3)) quantize_tail(x, y, n4 * 4 + threadIdx.x, s_tensor);
 }
 
-// Scalar path: any alignment, any per-axis layout, and the vector tail.
+// Per-axis paths.  Both take four consecutive elements of the flat tensor per
+// access (x 16-byte, y 4-byte aligned whatever the shape) and find their
+// scales; one element at a time, with two 64-bit divisions each, a 4096 x
+// 11008 weight with a scale per column took 107 us (now 41 us) and a 11007
+// x 4095 one with a scale per row 98 us (now 39 us).
+//
+// A scale per last-axis element (inner == 1): the scales of a group of four
+// repeat every Lq groups (Lq = axis_len / 4, / 2 or axis_len groups, by
+// axis_len % 4), so a thread whose stride T is a multiple of Lq keeps its
+// four reciprocals.
+constexpr int kUc = 4;
+
+__global__ __launch_bounds__(kThreads) void k_quantize_cols(const float *__restrict__ x, uint8_t *__restrict__ y,
+                                                            int64_t n, uint32_t Lq, int64_t T, uint32_t axis_len,
+                                                            const float *__restrict__ scale) {
+    const int64_t t = (int64_t)blockIdx.x * kThreads + threadIdx.x, n4 = n >> 2;
+    if (t < (n & 3)) quantize_tail(x, y, n4 * 4 + t, scale[(n4 * 4 + t) % axis_len]);
+    if (t >= T) return;
+    const f4 *x4 = reinterpret_cast<const f4 *>(x);
+    uint32_t *y4 = reinterpret_cast<uint32_t *>(y);
+    const uint32_t e0 = (uint32_t)t % Lq * 4;
+    Recip d[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) d[e] = make_recip(scale[(e0 + e) % axis_len]);
+    auto run = [&](auto fast) {
+        auto q = [&](float v, const Recip &r) {
+            if constexpr (decltype(fast)::value)
+                return div_fast(v, r);
+            else
+                return __fdiv_rn(v, r.s);
+        };
+        for (int64_t i0 = t; i0 < n4; i0 += T * kUc) {
+            f4 v[kUc];
+#pragma unroll
+            for (int u = 0; u < kUc; ++u) {
+                const int64_t i = i0 + u * T;
+                v[u] = i < n4 ? __builtin_nontemporal_load(x4 + i) : f4{0.f, 0.f, 0.f, 0.f};
+            }
+#pragma unroll
+            for (int u = 0; u < kUc; ++u) {
+                const int64_t i = i0 + u * T;
+                const uint32_t code = e4m3x2_hw(q(v[u].x, d[0]), q(v[u].y, d[1])) |
+                                      (e4m3x2_hw(q(v[u].z, d[2]), q(v[u].w, d[3])) << 16);
+                if (i < n4) y4[i] = code;
+            }
+        }
+    };
+    if (__builtin_amdgcn_ballot_w64(!(d[0].fast && d[1].fast && d[2].fast && d[3].fast)) == 0)
+        run(std::true_type{});
+    else
+        run(std::false_type{});
+}
+
+// Any other axis: the first element's place by one 32-bit division (n below
+// 2^32), the others by counting; the reciprocal changes where a group
+// crosses into the next scale's run.
+__global__ __launch_bounds__(kThreads) void k_quantize_axis(const float *__restrict__ x, uint8_t *__restrict__ y,
+                                                            int64_t n, uint32_t axis_len, uint32_t inner, int wraps,
+                                                            const float *__restrict__ scale) {
+    const f4 *x4 = reinterpret_cast<const f4 *>(x);
+    uint32_t *y4 = reinterpret_cast<uint32_t *>(y);
+    const int64_t n4 = n >> 2, stride = (int64_t)gridDim.x * kThreads * kUc;
+    auto place = [&](uint32_t e, uint32_t &a, uint32_t &rem) {
+        a = e / inner;
+        rem = e - a * inner;
+        if (wraps) a %= axis_len;
+    };
+    for (int64_t i0 = (int64_t)blockIdx.x * kThreads * kUc + threadIdx.x; i0 < n4; i0 += stride) {
+        f4 v[kUc];
+        float s[kUc];
+        uint32_t a[kUc], rem[kUc];
+#pragma unroll
+        for (int u = 0; u < kUc; ++u) {
+            const int64_t i = i0 + (int64_t)u * kThreads;
+            v[u] = i < n4 ? __builtin_nontemporal_load(x4 + i) : f4{0.f, 0.f, 0.f, 0.f};
+            place(i < n4 ? (uint32_t)i * 4 : 0u, a[u], rem[u]);
+            s[u] = scale[a[u]];
+        }
+#pragma unroll
+        for (int u = 0; u < kUc; ++u) {
+            const int64_t i = i0 + (int64_t)u * kThreads;
+            Recip d = make_recip(s[u]);
+            float q[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if (e && ++rem[u] == inner) {
+                    rem[u] = 0;
+                    a[u] = a[u] + 1 == axis_len ? 0 : a[u] + 1;
+                    d = make_recip(scale[a[u]]);
+                }
+                q[e] = div_by(v[u][e], d);
+            }
+            if (i < n4) y4[i] = e4m3x2_hw(q[0], q[1]) | (e4m3x2_hw(q[2], q[3]) << 16);
+        }
+    }
+    if (blockIdx.x == 0 && threadIdx.x < (n & 3)) {
+        uint32_t at, rt;
+        place((uint32_t)n4 * 4 + threadIdx.x, at, rt);
+        quantize_tail(x, y, n4 * 4 + threadIdx.x, scale[at]);
+    }
+}
+
+// Scalar path: any alignment and size.
 template <bool FROM_AMAX>
 __global__ __launch_bounds__(kThreads) void k_quantize_scalar(const float *__restrict__ x,
-                                                              uint8_t *__restrict__ y, int64_t begin,
-                                                              int64_t n, int64_t axis_len, int64_t inner,
+                                                              uint8_t *__restrict__ y, int64_t n,
+                                                              int64_t axis_len, int64_t inner,
                                                               const float *__restrict__ scale,
                                                               const uint32_t *__restrict__ part, int npart,
                                                               float *__restrict__ scale_out) {
@@ -102,7 +201,7 @@ __global__ __launch_bounds__(kThreads) void k_quantize_scalar(const float *__res
     int64_t stride = (int64_t)gridDim.x * kThreads;
     float s_amax = FROM_AMAX ? scale_from_partials<kThreads>(part, npart, red) : 0.0f;
     if (FROM_AMAX && scale_out && blockIdx.x == 0 && threadIdx.x == 0) *scale_out = s_amax;
-    for (int64_t i = begin + (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += stride) {
+    for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += stride) {
         float s = FROM_AMAX ? s_amax : scale[axis_len == 1 ? 0 : (i / inner) % axis_len];
         y[i] = (uint8_t)e4m3_encode(__fdiv_rn(x[i], s));
     }
@@ -117,19 +216,22 @@ __device__ inline void dec4(uint32_t w, float s, f4 &o) {
     o.x = lo.x * s; o.y = lo.y * s; o.z = hi.x * s; o.w = hi.y * s;
 }
 
+__device__ inline void dequantize_tail(const uint8_t *q, float *y, int64_t i, float s) {
+    const f2 v = __builtin_amdgcn_cvt_pk_f32_fp8((int)q[i], false);
+    y[i] = v.x * s;
+}
+
 // Same shape as k_quantize_vec with kUd 32-bit code words per thread,
-// kThreads apart; requires q 4-byte and y 16-byte aligned, inner % 4 == 0
-// per axis.
+// kThreads apart; requires q 4-byte and y 16-byte aligned.
 constexpr int kUd = 8;
 
 __global__ __launch_bounds__(kThreads) void k_dequantize_vec(const uint8_t *__restrict__ q,
-                                                             float *__restrict__ y, int64_t n4,
-                                                             int64_t axis_len, int64_t inner,
+                                                             float *__restrict__ y, int64_t n,
                                                              const float *__restrict__ scale) {
     const uint32_t *q4 = reinterpret_cast<const uint32_t *>(q);
     f4 *y4 = reinterpret_cast<f4 *>(y);
-    const float s_tensor = axis_len == 1 ? scale[0] : 0.0f;
-    const int64_t stride = (int64_t)gridDim.x * kThreads * kUd;
+    const float s = scale[0];
+    const int64_t n4 = n >> 2, stride = (int64_t)gridDim.x * kThreads * kUd;
     for (int64_t i0 = (int64_t)blockIdx.x * kThreads * kUd + threadIdx.x; i0 < n4; i0 += stride) {
         uint32_t w[kUd];
 #pragma unroll
@@ -140,20 +242,97 @@ __global__ __launch_bounds__(kThreads) void k_dequantize_vec(const uint8_t *__re
 #pragma unroll
         for (int u = 0; u < kUd; ++u) {
             const int64_t i = i0 + (int64_t)u * kThreads;
-            const float sc = axis_len == 1 ? s_tensor : scale[((i * 4) / inner) % axis_len];
             f4 o;
-            dec4(w[u], sc, o);
+            dec4(w[u], s, o);
             if (i < n4) y4[i] = o;
+        }
+    }
+    if (blockIdx.x == 0 && threadIdx.x < (n & 3)) dequantize_tail(q, y, n4 * 4 + threadIdx.x, s);
+}
+
+// k_quantize_cols and k_quantize_axis the other way
+__global__ __launch_bounds__(kThreads) void k_dequantize_cols(const uint8_t *__restrict__ q, float *__restrict__ y,
+                                                              int64_t n, uint32_t Lq, int64_t T, uint32_t axis_len,
+                                                              const float *__restrict__ scale) {
+    const int64_t t = (int64_t)blockIdx.x * kThreads + threadIdx.x, n4 = n >> 2;
+    if (t < (n & 3)) dequantize_tail(q, y, n4 * 4 + t, scale[(n4 * 4 + t) % axis_len]);
+    if (t >= T) return;
+    const uint32_t *q4 = reinterpret_cast<const uint32_t *>(q);
+    f4 *y4 = reinterpret_cast<f4 *>(y);
+    const uint32_t e0 = (uint32_t)t % Lq * 4;
+    float s[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) s[e] = scale[(e0 + e) % axis_len];
+    for (int64_t i0 = t; i0 < n4; i0 += T * kUc) {
+        uint32_t w[kUc];
+#pragma unroll
+        for (int u = 0; u < kUc; ++u) {
+            const int64_t i = i0 + u * T;
+            w[u] = i < n4 ? __builtin_nontemporal_load(q4 + i) : 0u;
+        }
+#pragma unroll
+        for (int u = 0; u < kUc; ++u) {
+            const int64_t i = i0 + u * T;
+            const f2 lo = __builtin_amdgcn_cvt_pk_f32_fp8((int)w[u], false);
+            const f2 hi = __builtin_amdgcn_cvt_pk_f32_fp8((int)w[u], true);
+            if (i < n4) y4[i] = f4{lo.x * s[0], lo.y * s[1], hi.x * s[2], hi.y * s[3]};
         }
     }
 }
 
+__global__ __launch_bounds__(kThreads) void k_dequantize_axis(const uint8_t *__restrict__ q, float *__restrict__ y,
+                                                              int64_t n, uint32_t axis_len, uint32_t inner, int wraps,
+                                                              const float *__restrict__ scale) {
+    const uint32_t *q4 = reinterpret_cast<const uint32_t *>(q);
+    f4 *y4 = reinterpret_cast<f4 *>(y);
+    const int64_t n4 = n >> 2, stride = (int64_t)gridDim.x * kThreads * kUc;
+    auto place = [&](uint32_t e, uint32_t &a, uint32_t &rem) {
+        a = e / inner;
+        rem = e - a * inner;
+        if (wraps) a %= axis_len;
+    };
+    for (int64_t i0 = (int64_t)blockIdx.x * kThreads * kUc + threadIdx.x; i0 < n4; i0 += stride) {
+        uint32_t w[kUc], a[kUc], rem[kUc];
+        float s[kUc];
+#pragma unroll
+        for (int u = 0; u < kUc; ++u) {
+            const int64_t i = i0 + (int64_t)u * kThreads;
+            w[u] = i < n4 ? __builtin_nontemporal_load(q4 + i) : 0u;
+            place(i < n4 ? (uint32_t)i * 4 : 0u, a[u], rem[u]);
+            s[u] = scale[a[u]];
+        }
+#pragma unroll
+        for (int u = 0; u < kUc; ++u) {
+            const int64_t i = i0 + (int64_t)u * kThreads;
+            const f2 lo = __builtin_amdgcn_cvt_pk_f32_fp8((int)w[u], false);
+            const f2 hi = __builtin_amdgcn_cvt_pk_f32_fp8((int)w[u], true);
+            f4 o = {lo.x, lo.y, hi.x, hi.y};
+            float se = s[u];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if (e && ++rem[u] == inner) {
+                    rem[u] = 0;
+                    a[u] = a[u] + 1 == axis_len ? 0 : a[u] + 1;
+                    se = scale[a[u]];
+                }
+                o[e] *= se;
+            }
+            if (i < n4) y4[i] = o;
+        }
+    }
+    if (blockIdx.x == 0 && threadIdx.x < (n & 3)) {
+        uint32_t at, rt;
+        place((uint32_t)n4 * 4 + threadIdx.x, at, rt);
+        dequantize_tail(q, y, n4 * 4 + threadIdx.x, scale[at]);
+    }
+}
+
 __global__ __launch_bounds__(kThreads) void k_dequantize_scalar(const uint8_t *__restrict__ q,
-                                                                float *__restrict__ y, int64_t begin,
-                                                                int64_t n, int64_t axis_len, int64_t inner,
+                                                                float *__restrict__ y, int64_t n,
+                                                                int64_t axis_len, int64_t inner,
                                                                 const float *__restrict__ scale) {
     int64_t stride = (int64_t)gridDim.x * kThreads;
-    for (int64_t i = begin + (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += stride) {
+    for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += stride) {
         float s = scale[axis_len == 1 ? 0 : (i / inner) % axis_len];
         f2 v = __builtin_amdgcn_cvt_pk_f32_fp8((int)q[i], false);
         y[i] = v.x * s;
@@ -227,14 +406,15 @@ __global__ __launch_bounds__(kAmaxThreads) void k_amax_partials(const float *__r
 // (4096x4096: 29.5 -> 26.6 us for both passes, 4096x11008: 67.8 -> 62.6 us,
 // bit-identical).  Each workgroup reduces the partial maxima to the scale
 // while its first loads are in flight.  Requires x 16-byte and y 4-byte
-// aligned, n % 4 == 0 (nv = n / 4 float4 groups).
+// aligned; the last n % 4 elements fall to workgroup 0.
 __global__ __launch_bounds__(kAmaxThreads) void k_quantize_after_amax(const float *__restrict__ x,
-                                                                     uint8_t *__restrict__ y, int64_t nv,
+                                                                     uint8_t *__restrict__ y, int64_t n,
                                                                      const uint32_t *__restrict__ part, int npart,
                                                                      float *__restrict__ scale_out) {
     __shared__ float red[kAmaxThreads / 64];
     const f4 *x4 = reinterpret_cast<const f4 *>(x);
     uint32_t *y4 = reinterpret_cast<uint32_t *>(y);
+    const int64_t nv = n >> 2;
     const int64_t stride = (int64_t)gridDim.x * kAmaxThreads * kAmaxU;
     const int64_t first = (int64_t)blockIdx.x * kAmaxThreads * kAmaxU + threadIdx.x;
     // this thread's last chunk of the amax pass's grid-stride walk (-1: none)
@@ -270,6 +450,7 @@ __global__ __launch_bounds__(kAmaxThreads) void k_quantize_after_amax(const floa
         run(std::true_type{});
     else
         run(std::false_type{});
+    if (blockIdx.x == 0 && threadIdx.x < (n & 3)) quantize_tail(x, y, nv * 4 + threadIdx.x, s_tensor);
 }
 
 __global__ void k_fill_u32(uint32_t *p, uint32_t v, int64_t n) {
@@ -292,8 +473,9 @@ constexpr int64_t kSmallMax = 65536;
 constexpr int kRedThreads = 1024;
 
 __global__ __launch_bounds__(kRedThreads) void k_quantize_dynamic_spread(
-    const float *__restrict__ x, uint8_t *__restrict__ y, int64_t n4, float *__restrict__ scale_out) {
+    const float *__restrict__ x, uint8_t *__restrict__ y, int64_t n, float *__restrict__ scale_out) {
     __shared__ float red[kRedThreads / 64];
+    const int64_t n4 = n >> 2;
     const f4 *x4 = reinterpret_cast<const f4 *>(x);
     float m = 0.0f;
     // 1024 threads x 16 float4 = the whole (at most 64K-element) tensor in
@@ -310,6 +492,7 @@ __global__ __launch_bounds__(kRedThreads) void k_quantize_dynamic_spread(
         m = absmax_acc(m, v[u].x); m = absmax_acc(m, v[u].y);
         m = absmax_acc(m, v[u].z); m = absmax_acc(m, v[u].w);
     }
+    if (threadIdx.x < (n & 3)) m = absmax_acc(m, x[n4 * 4 + threadIdx.x]);
     m = block_max<kRedThreads>(m, red);
     const float s = scale_from_amax_bits(f32_bits(m));
     const Recip d = make_recip(s);
@@ -321,10 +504,11 @@ __global__ __launch_bounds__(kRedThreads) void k_quantize_dynamic_spread(
         if ((int)blockIdx.x == u) mine = v[u];
     const int64_t i = (int64_t)blockIdx.x * kRedThreads + threadIdx.x;
     if (i < n4) reinterpret_cast<uint32_t *>(y)[i] = enc4(mine, d);
+    if (blockIdx.x == 0 && threadIdx.x < (n & 3)) quantize_tail(x, y, n4 * 4 + threadIdx.x, s);
     if (blockIdx.x == 0 && threadIdx.x == 0) *scale_out = s;
 }
 
-// Scalar fallback (unaligned pointers or n % 4 != 0): amax pass, then an
+// Scalar fallback (unaligned pointers): amax pass, then an
 // encode pass that re-reads x.
 __global__ __launch_bounds__(kSmallThreads) void k_quantize_dynamic_small(
     const float *__restrict__ x, uint8_t *__restrict__ y, int64_t n, float *__restrict__ scale_out) {
@@ -356,33 +540,67 @@ bool aligned4(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 3) == 0;
 
 }  // namespace
 
+namespace {
+
+// the stride of the cols kernels: whole periods of Lq groups, about kUc groups
+// per thread, at most 2048 workgroups (a longer period is one group's each)
+struct ColsPlan {
+    uint32_t Lq;
+    int64_t T;
+    unsigned grid;
+};
+ColsPlan plan_cols(int64_t n4, int64_t axis_len) {
+    ColsPlan p;
+    p.Lq = (uint32_t)(axis_len % 4 == 0 ? axis_len / 4 : axis_len % 2 == 0 ? axis_len / 2 : axis_len);
+    const int64_t per = (n4 + (int64_t)kUc * p.Lq - 1) / ((int64_t)kUc * p.Lq), cap = 2048 * kThreads / p.Lq;
+    const int64_t periods = per < cap ? per : cap;
+    p.T = (int64_t)p.Lq * (periods < 1 ? 1 : periods);
+    p.grid = (unsigned)((p.T + kThreads - 1) / kThreads);
+    return p;
+}
+
+}  // namespace
+
 hipError_t launch_quantize(const float *x, uint8_t *y, int64_t outer, int64_t axis_len,
                            int64_t inner, const float *scale, hipStream_t s) {
-    int64_t n = outer * axis_len * inner;
+    const int64_t n = outer * axis_len * inner;
     if (n == 0) return hipSuccess;
-    const bool quad_uniform = axis_len == 1 || inner % 4 == 0;
-    const int64_t n4 = (aligned16(x) && aligned4(y) && quad_uniform) ? n / 4 : 0;
-    if (n4)
-        hipLaunchKernelGGL(k_quantize_vec<false>, dim3(grid_vec(n4, kU)), dim3(kThreads), 0, s, x, y, n4, axis_len,
-                           inner, scale, nullptr, 0, nullptr);
-    if (n4 * 4 < n)
-        hipLaunchKernelGGL(k_quantize_scalar<false>, dim3(grid_for(n - n4 * 4)), dim3(kThreads), 0, s, x, y,
-                           n4 * 4, n, axis_len, inner, scale, nullptr, 0, nullptr);
+    const bool vec = aligned16(x) && aligned4(y);
+    if (vec && axis_len == 1) {
+        hipLaunchKernelGGL(k_quantize_vec<false>, dim3(grid_vec(n / 4, kU)), dim3(kThreads), 0, s, x, y, n, scale,
+                           nullptr, 0, nullptr);
+    } else if (vec && inner == 1 && axis_len < ((int64_t)1 << 30)) {
+        const ColsPlan p = plan_cols(n / 4, axis_len);
+        hipLaunchKernelGGL(k_quantize_cols, dim3(p.grid), dim3(kThreads), 0, s, x, y, n, p.Lq, p.T, (uint32_t)axis_len,
+                           scale);
+    } else if (vec && n < ((int64_t)1 << 32)) {
+        hipLaunchKernelGGL(k_quantize_axis, dim3(grid_vec(n / 4, kUc)), dim3(kThreads), 0, s, x, y, n,
+                           (uint32_t)axis_len, (uint32_t)inner, outer > 1 ? 1 : 0, scale);
+    } else {
+        hipLaunchKernelGGL(k_quantize_scalar<false>, dim3(grid_for(n)), dim3(kThreads), 0, s, x, y, n,
+                           axis_len, inner, scale, nullptr, 0, nullptr);
+    }
     return hipGetLastError();
 }
 
 hipError_t launch_dequantize(const uint8_t *x, float *y, int64_t outer, int64_t axis_len,
                              int64_t inner, const float *scale, hipStream_t s) {
-    int64_t n = outer * axis_len * inner;
+    const int64_t n = outer * axis_len * inner;
     if (n == 0) return hipSuccess;
-    const bool quad_uniform = axis_len == 1 || inner % 4 == 0;
-    const int64_t n4 = (aligned4(x) && aligned16(y) && quad_uniform) ? n / 4 : 0;
-    if (n4)
-        hipLaunchKernelGGL(k_dequantize_vec, dim3(grid_vec(n4, kUd)), dim3(kThreads), 0, s, x, y, n4, axis_len, inner,
+    const bool vec = aligned4(x) && aligned16(y);
+    if (vec && axis_len == 1) {
+        hipLaunchKernelGGL(k_dequantize_vec, dim3(grid_vec(n / 4, kUd)), dim3(kThreads), 0, s, x, y, n, scale);
+    } else if (vec && inner == 1 && axis_len < ((int64_t)1 << 30)) {
+        const ColsPlan p = plan_cols(n / 4, axis_len);
+        hipLaunchKernelGGL(k_dequantize_cols, dim3(p.grid), dim3(kThreads), 0, s, x, y, n, p.Lq, p.T,
+                           (uint32_t)axis_len, scale);
+    } else if (vec && n < ((int64_t)1 << 32)) {
+        hipLaunchKernelGGL(k_dequantize_axis, dim3(grid_vec(n / 4, kUc)), dim3(kThreads), 0, s, x, y, n,
+                           (uint32_t)axis_len, (uint32_t)inner, outer > 1 ? 1 : 0, scale);
+    } else {
+        hipLaunchKernelGGL(k_dequantize_scalar, dim3(grid_for(n)), dim3(kThreads), 0, s, x, y, n, axis_len, inner,
                            scale);
-    if (n4 * 4 < n)
-        hipLaunchKernelGGL(k_dequantize_scalar, dim3(grid_for(n - n4 * 4)), dim3(kThreads), 0, s, x, y, n4 * 4, n,
-                           axis_len, inner, scale);
+    }
     return hipGetLastError();
 }
 
@@ -425,12 +643,12 @@ hipError_t launch_amax_to_float(const uint32_t *amax_bits, float *out, hipStream
 hipError_t launch_quantize_dynamic(const float *x, uint8_t *y, int64_t n, float *scale_out,
                                    uint32_t *work, hipStream_t s) {
     if (n <= kSmallMax) {
-        if (n % 4 == 0 && aligned16(x) && (reinterpret_cast<uintptr_t>(y) & 3) == 0) {
+        if (aligned16(x) && aligned4(y)) {
             // one float4 per thread in the encode pass: ceil(n4 / 1024) <= 16 workgroups
             const int64_t n4 = n / 4;
             int p = (int)((n4 + kRedThreads - 1) / kRedThreads);
             p = p < 1 ? 1 : p;
-            hipLaunchKernelGGL(k_quantize_dynamic_spread, dim3(p), dim3(kRedThreads), 0, s, x, y, n4, scale_out);
+            hipLaunchKernelGGL(k_quantize_dynamic_spread, dim3(p), dim3(kRedThreads), 0, s, x, y, n, scale_out);
         } else
             hipLaunchKernelGGL(k_quantize_dynamic_small, dim3(1), dim3(kSmallThreads), 0, s, x, y, n,
                                scale_out);
@@ -441,8 +659,8 @@ hipError_t launch_quantize_dynamic(const float *x, uint8_t *y, int64_t n, float 
     int npart = 0;
     hipError_t err = launch_amax_partials(x, n, work, &npart, s);
     if (err != hipSuccess) return err;
-    if (n % 4 == 0 && aligned16(x) && aligned4(y)) {
-        hipLaunchKernelGGL(k_quantize_after_amax, dim3((unsigned)npart), dim3(kAmaxThreads), 0, s, x, y, n / 4, work,
+    if (aligned16(x) && aligned4(y)) {
+        hipLaunchKernelGGL(k_quantize_after_amax, dim3((unsigned)npart), dim3(kAmaxThreads), 0, s, x, y, n, work,
                            npart, scale_out);
         return hipGetLastError();
     }
@@ -451,13 +669,12 @@ hipError_t launch_quantize_dynamic(const float *x, uint8_t *y, int64_t n, float 
 
 hipError_t launch_quantize_dynamic_parts(const float *x, uint8_t *y, int64_t n, const uint32_t *part, int npart,
                                          float *scale_out, hipStream_t s) {
-    const int64_t n4 = (aligned16(x) && aligned4(y)) ? n / 4 : 0;
-    if (n4)
-        hipLaunchKernelGGL(k_quantize_vec<true>, dim3(grid_vec(n4, kU)), dim3(kThreads), 0, s, x, y, n4, (int64_t)1,
-                           n, nullptr, part, npart, scale_out);
-    if (n4 * 4 < n)
-        hipLaunchKernelGGL(k_quantize_scalar<true>, dim3(grid_for(n - n4 * 4)), dim3(kThreads), 0, s, x, y,
-                           n4 * 4, n, (int64_t)1, n, nullptr, part, npart, n4 ? nullptr : scale_out);
+    if (aligned16(x) && aligned4(y))
+        hipLaunchKernelGGL(k_quantize_vec<true>, dim3(grid_vec(n / 4, kU)), dim3(kThreads), 0, s, x, y, n, nullptr,
+                           part, npart, scale_out);
+    else
+        hipLaunchKernelGGL(k_quantize_scalar<true>, dim3(grid_for(n)), dim3(kThreads), 0, s, x, y, n,
+                           (int64_t)1, n, nullptr, part, npart, scale_out);
     return hipGetLastError();
 }
 

@@ -1,0 +1,74 @@
+"""Quantize / dequantize with a scale per axis element, dynamic quantisation of
+odd sizes and packing of [N, K] weights: equal to the oracle byte for byte at
+the remainders of the four-element accesses, in every layout of the axis."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from luisaml_amd import capi, synth
+
+pytestmark = pytest.mark.gpu
+
+
+def special(x):
+    f = x.reshape(-1)
+    for i, v in enumerate([np.nan, np.inf, -np.inf, 0.0, -0.0, 1e-40, 3e38]):
+        f[(i * 7919) % f.size] = v
+    return x
+
+
+# shape, axis: the last axis with lengths 0..3 mod 4 (periods of one, two and
+# four rows), fewer and more rows than a period, more groups than the grid; an
+# inner run of 1, 2, 3, more and odd, outer repeats; n below 4
+SHAPES = [((5, 8), 1), ((9, 1000), 1), ((7, 1002), 1), ((13, 1001), 1), ((1, 3), 1), ((2, 5003), 1), ((3000, 2051), 1),
+          ((17, 1), 0), ((1001, 7), 0), ((33, 1023), 0), ((64, 4095), 0), ((2, 3), 0), ((3, 5, 2), 1), ((4, 6, 9), 1),
+          ((2, 3, 7, 13), 1), ((3, 130, 4), 1), ((3, 4, 11, 5), 2), ((2100, 2051), 0)]
+
+
+@pytest.mark.parametrize("shape,axis", SHAPES)
+@pytest.mark.parametrize("shift", [0, 1])
+def test_per_axis(dev, shape, axis, shift):
+    x = special(synth.normal(sum(shape), shape))
+    s = np.abs(synth.normal(axis + 1, (shape[axis],), std=0.05)) + np.float32(1e-4)
+    s[0] = 1e-25  # outside the reciprocal's range
+    n = x.size
+    xb = torch.empty(n + shift, device=dev)
+    yb = torch.empty(n + shift, dtype=torch.uint8, device=dev)
+    dx, q = xb[shift:].view(shape), yb[shift:].view(shape)
+    dx.copy_(torch.from_numpy(x))
+    capi.quantize(dx, torch.from_numpy(s).to(dev), axis=axis, out=q)
+    ref = oracle.quantize(x, s, axis=axis)
+    assert np.array_equal(q.cpu().numpy(), ref)
+    back = capi.dequantize(q, torch.from_numpy(s).to(dev), axis=axis, out=xb[shift:].view(shape))
+    assert np.array_equal(back.cpu().numpy(), oracle.dequantize(ref, s, axis=axis), equal_nan=True)
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 4097, 16387, 65533, 65537, 262147, 2097155, 9000001])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_dynamic_odd_sizes(dev, n, shift):
+    """The largest magnitude in the last element, so the tail sets the scale."""
+    x = synth.normal(n, (n,))
+    x[-1] = -9.0
+    buf = torch.empty(n + shift, device=dev)
+    buf[shift:].copy_(torch.from_numpy(x))
+    q, s = capi.quantize_dynamic(buf[shift:])
+    ref = oracle.dynamic_scale(x)
+    assert float(s.item()) == ref
+    assert np.array_equal(q.cpu().numpy(), oracle.quantize(x, ref))
+    back = capi.dequantize(q, s)
+    assert np.array_equal(back.cpu().numpy(), oracle.dequantize(oracle.quantize(x, ref), ref))
+
+
+@pytest.mark.parametrize("N,K", [(1, 1), (3, 15), (65, 16), (64, 17), (130, 255), (70, 1001), (33, 128), (5, 4099)])
+@pytest.mark.parametrize("shift", [0, 1, 2, 3])
+def test_pack_nk_bytes(dev, N, K, shift):
+    w = (np.arange(N * K, dtype=np.int64) * 2654435761 >> 7).astype(np.uint8).reshape(N, K)
+    buf = torch.empty(N * K + shift, dtype=torch.uint8, device=dev)
+    buf[shift:].copy_(torch.from_numpy(w.reshape(-1)))
+    p = capi.pack_weight(buf[shift:].view(N, K), True).cpu().numpy()
+    Kp, Np = -(-K // 128) * 128, -(-N // 64) * 64
+    full = np.zeros((Np, Kp), np.uint8)
+    full[:N, :K] = w
+    ref = full.reshape(Np // 64, 64, Kp // 16, 16).transpose(0, 2, 1, 3).reshape(-1)
+    assert np.array_equal(p, ref)
