@@ -99,7 +99,7 @@ __device__ inline v8i join(u4 lo, u4 hi) {
 typedef float f4 __attribute__((ext_vector_type(4)));
 
 // SB (DYN only): activation slots of 4 floats per lane per K block, at least
-// ceil(M/2).  ONE (DYN only; 0, 4 or 8): nonzero when every wavefront's K
+// ceil(M/2).  ONE (DYN only; 0, 4, 8 or 16): nonzero when every wavefront's K
 // blocks fit ONE slots, so that one round of ONE activation loads serves
 // both the amax and the encode (4 where they fit: at M <= 2 and K <= 4096
 // the four empty slots of an 8-slot round cost 0.1 us per launch).
@@ -116,9 +116,9 @@ template <int NB, int MB, int WAVES, int UNROLL, bool EXACT, bool DYN, int SB = 
 __global__ __launch_bounds__(WAVES * 64) void k_gemm_skinny(const uint8_t *bp, const void *src, int ld, int M, int K,
                                                             int kc, int nkb, int rg, SkinnyArgs g) {
     static_assert(!DYN || MB == 1, "the fused quantiser serves M <= 16");
-    static_assert(NB == 4, "a workgroup reads one whole 64-column panel");
-    static_assert(!DYN || (SB >= 1 && SB <= 8 && LCML_SKINNY_PF == 1 && UNROLL == 1),
-                  "the fused quantiser: M <= 2*SB <= 16, one K block per load");
+    static_assert(NB == 4 || ((NB == 1 || NB == 2) && MB == 1), "16-column blocks of one panel");
+    static_assert(!DYN || (SB >= 1 && SB <= 8 && LCML_SKINNY_PF == 1 && (UNROLL == 1 || NB < 4)),
+                  "the fused quantiser: M <= 2*SB <= 16, one K block per load of a whole panel");
     constexpr int NT = WAVES * 64;
     // the wavefronts' partial tiles, register r of lane l of block j at
     // [w][j][r][l]: the epilogue's lanes read consecutive words (no bank
@@ -174,7 +174,8 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_skinny(const uint8_t *bp, c
     // K block's first byte.
     const __amdgpu_buffer_rsrc_t b_rsrc = __builtin_amdgcn_make_buffer_rsrc(
         (void *)(bp + (size_t)(blk0 >> 2) * (size_t)kc * 1024), 0, kc * 1024, kRsrcFlags);
-    const uint32_t b_lane = (uint32_t)(lane & 15) * 16u + (uint32_t)(lane >> 4) * 2048u;
+    const uint32_t b_lane =
+        (uint32_t)(lane & 15) * 16u + (uint32_t)(lane >> 4) * 2048u + (NB < 4 ? (uint32_t)(blk0 & 3) * 256u : 0u);
     // activations (E4M3, without DYN): row lane%16, k offset (lane/16)*32 of a K block
     const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(
         DYN ? nullptr : const_cast<void *>(src), 0, DYN ? 0 : (int)((int64_t)(M - 1) * ld + K), kRsrcFlags);
@@ -328,7 +329,7 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_skinny(const uint8_t *bp, c
         }
     };
     f4 v[UQ];
-    static_assert(!ONE || (DYN && (ONE == 4 || ONE == 8) && UQ % SB == 0), "one round: whole blocks of slots");
+    static_assert(!ONE || (DYN && (ONE == 4 || ONE == 8 || (ONE == 16 && NB < 4)) && UQ % SB == 0), "one round: whole blocks of slots");
     if constexpr (ONE) {
         // slot u holds slot u%SB of block kb_begin + u/SB (the per-block
         // layout above): the amax reads these registers, and the encode
@@ -346,8 +347,10 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_skinny(const uint8_t *bp, c
     } else if constexpr (DYN) {
 #pragma unroll
         for (int u = 0; u < UQ; ++u) v[u] = xq(u * NT + tid);
-        xload_block(xb0, kb_begin);
-        xload_block(xb1, kb_begin + 1);
+        if constexpr (NB == 4) {
+            xload_block(xb0, kb_begin);
+            xload_block(xb1, kb_begin + 1);
+        }
         __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
@@ -379,7 +382,7 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_skinny(const uint8_t *bp, c
     // DYN: a second K block in flight while the scale is computed (issued
     // after the scale prefetch: before it, 0.1 us slower at M = 1 and 4)
     Frag fx;
-    if constexpr (DYN) {
+    if constexpr (DYN && NB == 4) {
         load(fx, kb_begin + 1);
         __builtin_amdgcn_sched_barrier(0);
     }
@@ -400,7 +403,8 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_skinny(const uint8_t *bp, c
             const int nslot = ONE ? (kb_end - kb_begin) * SB : UQ;
 #pragma unroll
             for (int u = 0; u < UQ; ++u) {
-                if (u >= nslot) break;
+                // (16 slots: no way out, or the loop stays rolled and v in scratch)
+                if (ONE != 16 && u >= nslot) break;
                 // zeros past the end; NaN compares false and is skipped, as
                 // in the standalone amax
                 const float ax = fabsf(v[u].x), ay = fabsf(v[u].y), az = fabsf(v[u].z), aw = fabsf(v[u].w);
@@ -436,23 +440,22 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_skinny(const uint8_t *bp, c
     // copy (rows below M; columns past K get the zeros x holds there).  Only
     // this wavefront reads them, and a wavefront's LDS accesses take effect
     // in order, so no barrier is needed.
-    auto encode_block = [&](const f4 *xb, int kb) {
-        if (kb >= kb_end) return;
-        auto run = [&](auto mode) {
+    auto encode_slots = [&](const f4 *xb, int kb, auto mode) {
 #pragma unroll
-            for (int sl = 0; sl < SB; ++sl) {
-                const uint32_t r = 2 * sl + (lane >> 5), c = (uint32_t)kb * 32 + (lane & 31);
-                if (r < (uint32_t)M) {
-                    const f4 x4 = xb[sl];
-                    uint32_t code;
-                    if constexpr (decltype(mode)::value == 2)
-                        code = quantize4_clean(x4.x, x4.y, x4.z, x4.w, d);
-                    else
-                        code = quantize4_t<decltype(mode)::value == 1>(x4.x, x4.y, x4.z, x4.w, d);
-                    reinterpret_cast<uint32_t *>(a_lds + r * pitch)[c] = code;
-                }
+        for (int sl = 0; sl < SB; ++sl) {
+            const uint32_t r = 2 * sl + (lane >> 5), c = (uint32_t)kb * 32 + (lane & 31);
+            if (r < (uint32_t)M) {
+                const f4 x4 = xb[sl];
+                uint32_t code;
+                if constexpr (decltype(mode)::value == 2)
+                    code = quantize4_clean(x4.x, x4.y, x4.z, x4.w, d);
+                else
+                    code = quantize4_t<decltype(mode)::value == 1>(x4.x, x4.y, x4.z, x4.w, d);
+                reinterpret_cast<uint32_t *>(a_lds + r * pitch)[c] = code;
             }
-        };
+        }
+    };
+    auto by_mode = [&](auto run) {
         if (enc_mode == 2)
             run(std::integral_constant<int, 2>{});
         else if (enc_mode == 1)
@@ -460,7 +463,35 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_skinny(const uint8_t *bp, c
         else
             run(std::integral_constant<int, 0>{});
     };
-    if constexpr (ONE) {
+    auto encode_block = [&](const f4 *xb, int kb) {
+        if (kb >= kb_end) return;
+        by_mode([&](auto mode) { encode_slots(xb, kb, mode); });
+    };
+    if constexpr (DYN && NB < 4) {
+        // UNROLL blocks of weights are in flight: all of this wavefront's
+        // activations are encoded now, then its blocks run in groups
+        if constexpr (ONE) {
+            by_mode([&](auto mode) {
+#pragma unroll
+                for (int b = 0; b < UQ / SB; ++b)
+                    if (kb_begin + b < kb_end) encode_slots(v + b * SB, kb_begin + b, mode);
+            });
+        } else {
+            for (int kb = kb_begin; kb < kb_end; kb += 2) {
+                xload_block(xb0, kb);
+                xload_block(xb1, kb + 1);
+                encode_block(xb0, kb);
+                encode_block(xb1, kb + 1);
+            }
+        }
+        for (int kb0 = kb_begin; kb0 < kb_end; kb0 += UNROLL) {
+            read_a(fr[0], kb0);
+            compute(fr[0], kb0);
+            __builtin_amdgcn_sched_barrier(0);
+            load(fr[0], kb0 + UNROLL);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    } else if constexpr (ONE) {
         // the next block's activations are always v[0..SB-1]: after its
         // encode the slots move down by SB
         auto encode_v = [&](int kb) {
@@ -620,6 +651,18 @@ int skinny_row_blocks(int64_t M, int64_t N, int64_t K, double *cost) {
     return mb;
 }
 
+// 16-column blocks per workgroup for M <= 16: the whole panel where the panels
+// give more than half the CUs a workgroup, else half of it or a quarter, with
+// two or four K blocks per load, so that as many bytes are in flight per
+// wavefront and the weights stream through more CUs.  N = 4096 (a quarter),
+// E4M3 in, whole panels -> now: K = 4096 M = 1 7.7 -> 5.5 us, M = 16
+// 8.9 -> 6.6; K = 11008 16.3 -> 9.7 and 19.7 -> 12.0; N = 6144 (half), K = 4096,
+// M = 1 9.2 -> 6.9.
+int skinny_col_blocks(int64_t N) {
+    const int64_t panels = (N + 63) / 64;
+    return panels > 128 ? 4 : panels > 64 ? 2 : 1;
+}
+
 hipError_t launch_gemm_skinny(int64_t M, int64_t N, int64_t K, const uint8_t *a, int64_t lda,
                               const uint8_t *bp, const Epilogue &e, bool exact, hipStream_t s) {
     // 32-bit buffer extents and kernel arguments (the C ABI checks the same)
@@ -637,21 +680,26 @@ hipError_t launch_gemm_skinny(int64_t M, int64_t N, int64_t K, const uint8_t *a,
     // row blocks of 16 per workgroup (every weight fragment feeds MB MFMAs),
     // and row groups of 16*MB rows beyond that
     const int mb = skinny_row_blocks(M, N, K, nullptr);
+    const int nb = mb == 1 ? skinny_col_blocks(N) : NB;
     g.rg = (int)((M + 16 * mb - 1) / (16 * mb));
-    const unsigned grid = (unsigned)((g.nblk16 + NB - 1) / NB * g.rg);
-#define LCML_SKINNY_LAUNCH(MBV)                                                                                  \
+    const unsigned grid = (unsigned)(((N + 15) / 16 + nb - 1) / nb * g.rg);
+#define LCML_SKINNY_LAUNCH(NBV, MBV, UV)                                                                         \
     if (exact)                                                                                                 \
-        hipLaunchKernelGGL((k_gemm_skinny<NB, MBV, W, U, true, false>), dim3(grid), dim3(W * 64), 0, s,          \
+        hipLaunchKernelGGL((k_gemm_skinny<NBV, MBV, W, UV, true, false>), dim3(grid), dim3(W * 64), 0, s,        \
                            LCML_SKINNY_LEAD(g, g.a, g.lda), g);                                                 \
     else                                                                                                       \
-        hipLaunchKernelGGL((k_gemm_skinny<NB, MBV, W, U, false, false>), dim3(grid), dim3(W * 64), 0, s,         \
+        hipLaunchKernelGGL((k_gemm_skinny<NBV, MBV, W, UV, false, false>), dim3(grid), dim3(W * 64), 0, s,       \
                            LCML_SKINNY_LEAD(g, g.a, g.lda), g)
-    if (mb == 1) {
-        LCML_SKINNY_LAUNCH(1);
+    if (nb == 1) {
+        LCML_SKINNY_LAUNCH(1, 1, 4);
+    } else if (nb == 2) {
+        LCML_SKINNY_LAUNCH(2, 1, 2);
+    } else if (mb == 1) {
+        LCML_SKINNY_LAUNCH(NB, 1, U);
     } else if (mb == 2) {
-        LCML_SKINNY_LAUNCH(2);
+        LCML_SKINNY_LAUNCH(NB, 2, U);
     } else {
-        LCML_SKINNY_LAUNCH(4);
+        LCML_SKINNY_LAUNCH(NB, 4, U);
     }
 #undef LCML_SKINNY_LAUNCH
     return hipGetLastError();
@@ -675,26 +723,38 @@ hipError_t launch_gemm_skinny_dynamic(int64_t M, int64_t N, int64_t K, const flo
     g.rg = 1;
     g.e = e;
     constexpr int NB = LCML_SKINNY_NB, W = LCML_SKINNY_WAVES, U = LCML_SKINNY_UNROLL;
-    const unsigned grid = (unsigned)((g.nblk16 + NB - 1) / NB);
+    const int nb = skinny_col_blocks(N);
+    const unsigned grid = (unsigned)(((N + 15) / 16 + nb - 1) / nb);
     const unsigned lds = (unsigned)skinny_dynamic_lds_bytes(M, K);
     // activation slots per lane per K block: ceil(M/2), rounded up to 1, 2,
     // 4, 8; one round of 4 or 8 activation loads when a wavefront's K blocks
     // (at most ceil(nkb / W)) take at most that many slots
-    auto run_one = [&](auto sb, auto one) -> hipError_t {
+    auto run_nb = [&](auto nbv, auto uv, auto sb, auto one) -> hipError_t {
+        constexpr int B = decltype(nbv)::value, UV = decltype(uv)::value;
         constexpr int SB = decltype(sb)::value;
         constexpr int ONE = decltype(one)::value;
-        const void *fn = exact ? reinterpret_cast<const void *>(k_gemm_skinny<NB, 1, W, U, true, true, SB, ONE>)
-                               : reinterpret_cast<const void *>(k_gemm_skinny<NB, 1, W, U, false, true, SB, ONE>);
+        const void *fn = exact ? reinterpret_cast<const void *>(k_gemm_skinny<B, 1, W, UV, true, true, SB, ONE>)
+                               : reinterpret_cast<const void *>(k_gemm_skinny<B, 1, W, UV, false, true, SB, ONE>);
         static std::atomic<uint64_t> lds_set[2];
         if (hipError_t err = ensure_dynamic_lds(fn, (int)kSkinnyDynLdsMax, lds_set[exact]); err != hipSuccess)
             return err;
         if (exact)
-            hipLaunchKernelGGL((k_gemm_skinny<NB, 1, W, U, true, true, SB, ONE>), dim3(grid), dim3(W * 64), lds, s,
+            hipLaunchKernelGGL((k_gemm_skinny<B, 1, W, UV, true, true, SB, ONE>), dim3(grid), dim3(W * 64), lds, s,
                                LCML_SKINNY_LEAD(g, g.x, g.ldx), g);
         else
-            hipLaunchKernelGGL((k_gemm_skinny<NB, 1, W, U, false, true, SB, ONE>), dim3(grid), dim3(W * 64), lds, s,
+            hipLaunchKernelGGL((k_gemm_skinny<B, 1, W, UV, false, true, SB, ONE>), dim3(grid), dim3(W * 64), lds, s,
                                LCML_SKINNY_LEAD(g, g.x, g.ldx), g);
         return hipGetLastError();
+    };
+    auto run_one = [&](auto sb, auto one) -> hipError_t {
+        using I1 = std::integral_constant<int, 1>;
+        using I2 = std::integral_constant<int, 2>;
+        if (nb == 1) return run_nb(I1{}, std::integral_constant<int, 4>{}, sb, one);
+        if (nb == 2) return run_nb(I2{}, I2{}, sb, one);
+        if constexpr (decltype(one)::value == 16)
+            return hipErrorInvalidValue;  // fewer than four column blocks only
+        else
+            return run_nb(std::integral_constant<int, NB>{}, std::integral_constant<int, U>{}, sb, one);
     };
     auto run = [&](auto sb) -> hipError_t {
         constexpr int SB = decltype(sb)::value;
@@ -702,6 +762,8 @@ hipError_t launch_gemm_skinny_dynamic(int64_t M, int64_t N, int64_t K, const flo
         if constexpr (SB <= 4)
             if (slots <= 4) return run_one(sb, std::integral_constant<int, 4>{});
         if (slots <= 8) return run_one(sb, std::integral_constant<int, 8>{});
+        if constexpr (SB <= 2)
+            if (slots <= 16 && nb < 4) return run_one(sb, std::integral_constant<int, 16>{});
         return run_one(sb, std::integral_constant<int, 0>{});
     };
     if (M <= 2) return run(std::integral_constant<int, 1>{});
