@@ -7,8 +7,9 @@ tree).  Flags:
   -Xclang -target-feature -Xclang -packed-fp32-ops
                                             no v_pk_{add,mul,fma}_f32 generation
   -fvisibility=hidden                       only the LCML_API C symbols export
-  -mllvm -amdgpu-kernarg-preload-count=N    (gemm_skinny.hip, gemm_w8a32.hip,
-                                            quantize.hip, gemv_valu.hip) the N leading scalar
+  -mllvm -amdgpu-kernarg-preload-count=N    (gemm_skinny.hip, gemm_rows.hip,
+                                            gemm_w8a32.hip, quantize.hip,
+                                            gemv_valu.hip) the N leading scalar
                                             kernel arguments arrive in SGPRs
                                             at wave start
 Usage:  python -m luisaml_amd.build   (or luisaml_amd.build.build())
@@ -45,6 +46,7 @@ COMMON = [
 EXTRA = {
     "gemm_skinny.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=8"],
     "quantize.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=4"],
+    "gemm_rows.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=7"],
     "gemm_w8a32.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=8"],
     "gemv_valu.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=6"],
 }

@@ -211,16 +211,34 @@ const char *kernel_label(int kernel) {
     }
 }
 
-int auto_gemm_kernel(int64_t M, int64_t N, int64_t K) {
-    if (M <= 16) return LCML_KERNEL_SKINNY;
+// AUTO's kernel and its modelled time in those units
+struct AutoChoice {
+    int kernel;
+    double units;
+};
+AutoChoice auto_gemm_choice(int64_t M, int64_t N, int64_t K) {
+    if (M <= 16) return {LCML_KERNEL_SKINNY, 0.0};
     const int64_t tiles = (M + 255) / 256 * ((N + 255) / 256);
-    if (tiles >= 256) return LCML_KERNEL_MFMA;
+    if (tiles >= 256) return {LCML_KERNEL_MFMA, 4.5 * (double)tiles / 256.0};
     double skinny = 0;
     lcml::skinny_row_blocks(M, N, K, &skinny);
     const double t128 = (double)((M + 127) / 128 * ((N + 127) / 128));
     const double small = 2.2 * (t128 > 256 ? t128 / 256 : 1.0);
-    if (skinny <= small && skinny < 4.5) return LCML_KERNEL_SKINNY;
-    return small < 4.5 ? LCML_KERNEL_MFMA_128 : LCML_KERNEL_MFMA;
+    if (skinny <= small && skinny < 4.5) return {LCML_KERNEL_SKINNY, skinny};
+    return small < 4.5 ? AutoChoice{LCML_KERNEL_MFMA_128, small} : AutoChoice{LCML_KERNEL_MFMA, 4.5};
+}
+
+int auto_gemm_kernel(int64_t M, int64_t N, int64_t K) { return auto_gemm_choice(M, N, K).kernel; }
+
+// Whether AUTO's dynamically quantised linear of M > 16 rows takes the codes
+// in 16-row blocks and the kernel that reads them: where that one's modelled
+// time is a seventh below the row-major choice's (19 us a unit at K = 4096, 3 us
+// besides; the 128x128 tiles often take that much less than their unit).  N =
+// 12288, K = 4096, with the quantiser: M = 100 31.7 us row-major against 28.1,
+// 256 43.1 against 43.4, 512 66 against 79.
+bool dynamic_by_rows(int64_t M, int64_t N, int64_t K) {
+    return M > 16 &&
+           lcml::gemm_rows_us(M, N, K) < 0.86 * (auto_gemm_choice(M, N, K).units * 19.0 * (double)K / 4096.0 + 3.0);
 }
 }  // namespace
 
@@ -403,6 +421,21 @@ int gemm_dynamic_impl(const char *fn, int64_t M, int64_t N, int64_t K, const flo
     uint8_t *q = ws;
     uint32_t *part = reinterpret_cast<uint32_t *>(ws + pad256(M * K));
     float *scale = x_scale_out ? x_scale_out : reinterpret_cast<float *>(ws + pad256(M * K) + LCML_FP8_DYNAMIC_WORKSPACE_BYTES);
+    if (kernel == LCML_KERNEL_AUTO && aligned(x, 16) && dynamic_by_rows(M, N, K)) {
+        // medium M: the codes in the layout of the GEMM that reads them
+        int npart = xa.npart;
+        if (!xa.part)
+            if (int rc = hip_status(lcml::launch_amax_partials(x, M * K, part, &npart, s), fn, "amax_partials")) return rc;
+        if (int rc = hip_status(lcml::launch_quantize_rows(x, q, M, K, xa.part ? xa.part : part, npart, scale, s), fn,
+                                "quantize_rows"))
+            return rc;
+        e.a_scale = scale;
+        if (int rc = hip_status(lcml::launch_gemm_rows(M, N, K, q, b_packed, e, s), fn, "gemm_rows")) return rc;
+        if (ya.part)
+            return hip_status(lcml::launch_amax_partials(static_cast<const float *>(y), M * N, ya.part, ya.npart, s),
+                              fn, "amax_partials");
+        return LCML_OK;
+    }
     hipError_t err = xa.part ? lcml::launch_quantize_dynamic_parts(x, q, M * K, xa.part, xa.npart, scale, s)
                              : lcml::launch_quantize_dynamic(x, q, M * K, scale, part, s);
     if (int rc = hip_status(err, fn, xa.part ? "quantize_dynamic_parts" : "quantize_dynamic")) return rc;

@@ -67,6 +67,14 @@ hipError_t launch_gemm_skinny(int64_t M, int64_t N, int64_t K, const uint8_t *a,
 // the skinny kernel's 16-row blocks per workgroup (1, 2 or 4) for an M x N
 // output over K, and its modelled time in units of one 4-block workgroup's run
 int skinny_row_blocks(int64_t M, int64_t N, int64_t K, double *cost);
+// medium M behind a dynamic quantisation (exact): codes in 16-row blocks
+// (M*K bytes), then the GEMM that reads them, and its modelled time in us (1e30
+// for sizes it does not take)
+double gemm_rows_us(int64_t M, int64_t N, int64_t K);
+hipError_t launch_quantize_rows(const float *x, uint8_t *y, int64_t M, int64_t K, const uint32_t *part, int npart,
+                                float *scale_out, hipStream_t s);
+hipError_t launch_gemm_rows(int64_t M, int64_t N, int64_t K, const uint8_t *a, const uint8_t *bp, const Epilogue &e,
+                            hipStream_t s);
 // fused DynamicQuantizeLinear + skinny GEMM (fp32 activations, M <= 16):
 // LDS use is skinny_dynamic_lds_bytes(M, K) <= kSkinnyDynLdsMax
 constexpr int64_t kSkinnyDynLdsMax = 128 * 1024 - 32 * 1024;

@@ -1,0 +1,80 @@
+"""Medium M behind a dynamic quantisation: codes in 16-row blocks, read by the
+kernel made for them, for each of its tile shapes and every remainder of the
+rows, columns and K.  The route depends on sizes alone, so the kernel trace says
+that it was taken; the scale is the oracle's, the sums are within its bound."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from luisaml_amd import capi, synth
+
+from .gemm_cases import assert_close
+
+pytestmark = pytest.mark.gpu
+
+
+ROWS_CASES = [(17, 1000, 1040), (32, 4096, 1040), (33, 2049, 2064), (47, 4100, 1168), (50, 6001, 1024), (63, 4096, 4112),
+              (64, 3000, 1936), (100, 4099, 2064), (100, 11008, 2048), (113, 12290, 2192), (129, 4096, 2064),
+              (200, 2050, 4096), (200, 4096, 2064), (250, 4096, 4112), (340, 4090, 2064), (384, 4096, 4096)]
+
+
+def case(dev, M, N, K):
+    x = synth.normal(M + K, (M, K))
+    x[M - 1, K - 1] = 7.0  # the last row of the last block sets the scale
+    w = synth.normal(N, (K, N), std=0.05)
+    sw = oracle.channel_scales(w, axis=1)
+    qw = oracle.quantize(w, sw, axis=1)
+    bias = synth.normal(3, (N,), std=0.01)
+    bp = capi.pack_weight(torch.from_numpy(qw).to(dev), False)
+    s = oracle.dynamic_scale(x)
+    ref, A, B = oracle.qlinear(oracle.quantize(x, s), s, qw, sw, bias=bias, act=oracle.ACT_RELU)
+    return x, bp, sw, bias, s, ref, oracle.gemm_abs_bound(A, B, bias)
+
+
+# 32x16 .. 96x64 tiles (by M and N), blocks of 1 to 16 rows at the end, odd N,
+# K one chunk over a 64-k quad, a 128-k block and the 8 parts
+@pytest.mark.parametrize("M,N,K", ROWS_CASES)
+def test_rows_match_oracle(dev, M, N, K):
+    x, bp, sw, bias, s, ref, bound = case(dev, M, N, K)
+    capi.kernel_trace()
+    sx = torch.empty(1, device=dev)
+    y, _ = capi.gemm_dynamic_ex(torch.from_numpy(x).to(dev), bp, torch.from_numpy(sw).to(dev), N, K,
+                                c=torch.from_numpy(bias).to(dev), act=capi.ACT_RELU, scale_out=sx)
+    assert capi.kernel_trace() == ["amax_partials", "quantize_rows", "gemm_rows"]
+    assert float(sx.item()) == s
+    assert_close(y.cpu().numpy(), ref, bound)
+
+
+def test_rows_partials_strides_and_alignment(dev):
+    """Partial maxima in and out as the other kernels'; an x that is not 16-byte
+    aligned keeps the row-major route; a row pitch of y above N; NaN and
+    infinite activations as the standalone quantiser gives them."""
+    M, N, K = 70, 2048, 1040
+    x, bp, sw, bias, s, ref, bound = case(dev, M, N, K)
+    d = [torch.from_numpy(v).to(dev) for v in (x, sw, bias)]
+    xp, yp = capi.amax_parts_buffer(M, K, dev), capi.amax_parts_buffer(M, N, dev)
+    xp.zero_()
+    xp[:2] = torch.tensor([1.0, float(np.abs(x).max())]).view(torch.int32).to(dev)
+    y, n = capi.gemm_dynamic_ex(d[0], bp, d[1], N, K, c=d[2], act=capi.ACT_RELU, x_amax=(xp, 2), y_amax_part=yp)
+    assert_close(y.cpu().numpy(), ref, bound)
+    assert yp[:n].cpu().view(torch.float32).max() == y.abs().max().cpu()
+    wide = torch.full((M, N + 8), 5.0, device=dev)
+    capi.gemm_dynamic(d[0], bp, d[1], N, K, c=d[2], act=capi.ACT_RELU, out=wide[:, :N])
+    assert torch.equal(wide[:, :N], y) and bool((wide[:, N:] == 5.0).all())
+    buf = torch.empty(M * K + 1, device=dev)
+    buf[1:].copy_(d[0].reshape(-1))
+    capi.kernel_trace()
+    y1 = capi.gemm_dynamic(buf[1:].view(M, K), bp, d[1], N, K, c=d[2], act=capi.ACT_RELU)
+    assert "gemm_rows" not in capi.kernel_trace()
+    assert_close(y1.cpu().numpy(), ref, bound)
+    for v in (np.nan, np.inf):
+        x2 = x.copy()
+        x2[69, 3] = v
+        d2 = torch.from_numpy(x2).to(dev)
+        q, s2 = capi.quantize_dynamic(d2)
+        a = capi.gemm(q, s2, bp, d[1], N, K).cpu().numpy()
+        b = capi.gemm_dynamic(d2, bp, d[1], N, K).cpu().numpy()
+        assert np.array_equal(np.isnan(a), np.isnan(b))
+        ok = ~np.isnan(a)
+        assert np.allclose(a[ok], b[ok], rtol=1e-4, atol=1e-5 * np.abs(a[ok]).max())
