@@ -414,19 +414,20 @@ __global__ __launch_bounds__(256) void k_conv2d_f32_mfma(ConvF32 a) {
         (void *)(a.x + ((int64_t)n * a.C + (int64_t)grp * cg) * HW), 0, cg * HW * 4, kRsrcFlags);
     // this lane's pixels
     const int p0 = (pt * 4 + wave) * 16 * PB + PB * (lane & 15);
-    int ih0[PB], iw0[PB], base[PB];
+    int ih0[PB], iw0[PB];
+    uint32_t base[PB];  // modulo 2^32, as the table's offsets: corners and taps may lie outside the image
 #pragma unroll
     for (int i = 0; i < PB; ++i) {
         const int p = p0 + i < OHW ? p0 + i : OHW - 1;
         const int oh = p / a.OW, ow = p - oh * a.OW;
         ih0[i] = oh * a.sh - a.ph;
         iw0[i] = ow * a.sw - a.pw;
-        base[i] = ih0[i] * a.W + iw0[i];
+        base[i] = (uint32_t)ih0[i] * (uint32_t)a.W + (uint32_t)iw0[i];
     }
     auto tap = [&](int i, int2 t) {  // pixel i's value under a table entry
         const int ih = ih0[i] + (t.y >> 16), iw = iw0[i] + (int)(int16_t)t.y;
         const bool ok = (uint32_t)ih < (uint32_t)a.H && (uint32_t)iw < (uint32_t)a.W;
-        return buf_f32(xr, ok ? (uint32_t)(base[i] + t.x) * 4u : kOOB);
+        return buf_f32(xr, ok ? (base[i] + (uint32_t)t.x) * 4u : kOOB);
     };
 
     f4 acc[PB][CB] = {};
@@ -437,7 +438,7 @@ __global__ __launch_bounds__(256) void k_conv2d_f32_mfma(ConvF32 a) {
             int2 t = {0, (int)0x80008000u};  // past K: a row above every image
             if (k < kn) {
                 const int tp = (kt + k) / cg, c = kt + k - tp * cg, kh = tp / a.KW, kw = tp - kh * a.KW;
-                t.x = c * HW + kh * a.dh * a.W + kw * a.dw;
+                t.x = (int)((uint32_t)c * (uint32_t)HW + (uint32_t)(kh * a.dh) * (uint32_t)a.W + (uint32_t)(kw * a.dw));
                 t.y = (int)((uint32_t)(kh * a.dh) << 16 | (uint32_t)(kw * a.dw));
             }
             tab[k] = t;
