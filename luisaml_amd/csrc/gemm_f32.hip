@@ -23,6 +23,9 @@ typedef float f2 __attribute__((ext_vector_type(2)));
 
 constexpr uint32_t kOOB = 0x80000000u;  // buffer offset past every extent: loads return zeros
 constexpr int kRsrcFlags = 0x00020000;  // raw buffer resource word 3
+// A launch of 2^32 work items in one dimension or more runs with that number
+// modulo 2^32 and reports no error: workgroups of 256 that a grid may have.
+constexpr int64_t kGridMax = ((int64_t)1 << 24) - 1;
 
 __device__ inline float buf_f32(__amdgpu_buffer_rsrc_t r, uint32_t off) {
     return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)off, 0, 0));
@@ -245,34 +248,34 @@ __global__ __launch_bounds__(256) void k_activation(const float *__restrict__ x,
 // from this chain only in fp32 rounding), begin pads only (conv.cpp:121),
 // dilation, groups, bias, activation.  For few output channels per group
 // (the matrix kernel would multiply mostly padding) and for geometries past
-// its 16- and 32-bit offsets.
+// its 16- and 32-bit offsets or its grid.
 __global__ __launch_bounds__(256) void k_conv2d_f32(const float *__restrict__ x, const float *__restrict__ w,
                                                     const float *__restrict__ bias, float *__restrict__ y, int C,
                                                     int H, int W, int Cout, int KH, int KW, int sh, int sw, int ph,
                                                     int pw, int dh, int dw, int group, int OH, int OW, int act,
                                                     int64_t total) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= total) return;
-    const int ow = (int)(i % OW);
-    const int oh = (int)((i / OW) % OH);
-    const int co = (int)((i / ((int64_t)OW * OH)) % Cout);
-    const int64_t n = i / ((int64_t)OW * OH * Cout);
-    const int cg = C / group, mg = Cout / group, g = co / mg;
-    const float *xn = x + (n * C + (int64_t)g * cg) * H * W;
-    const float *wc = w + (int64_t)co * cg * KH * KW;
-    float sum = 0.0f;
-    for (int kh = 0; kh < KH; ++kh) {
-        const int ih = oh * sh + kh * dh - ph;
-        if ((unsigned)ih >= (unsigned)H) continue;
-        for (int kw = 0; kw < KW; ++kw) {
-            const int iw = ow * sw + kw * dw - pw;
-            if ((unsigned)iw >= (unsigned)W) continue;
-            for (int c = 0; c < cg; ++c)
-                sum = fmaf(xn[((int64_t)c * H + ih) * W + iw], wc[((int64_t)c * KH + kh) * KW + kw], sum);
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
+        const int ow = (int)(i % OW);
+        const int oh = (int)((i / OW) % OH);
+        const int co = (int)((i / ((int64_t)OW * OH)) % Cout);
+        const int64_t n = i / ((int64_t)OW * OH * Cout);
+        const int cg = C / group, mg = Cout / group, g = co / mg;
+        const float *xn = x + (n * C + (int64_t)g * cg) * H * W;
+        const float *wc = w + (int64_t)co * cg * KH * KW;
+        float sum = 0.0f;
+        for (int kh = 0; kh < KH; ++kh) {
+            const int ih = oh * sh + kh * dh - ph;
+            if ((unsigned)ih >= (unsigned)H) continue;
+            for (int kw = 0; kw < KW; ++kw) {
+                const int iw = ow * sw + kw * dw - pw;
+                if ((unsigned)iw >= (unsigned)W) continue;
+                for (int c = 0; c < cg; ++c)
+                    sum = fmaf(xn[((int64_t)c * H + ih) * W + iw], wc[((int64_t)c * KH + kh) * KW + kw], sum);
+            }
         }
+        if (bias) sum += bias[co];
+        y[i] = apply_act(sum, act);
     }
-    if (bias) sum += bias[co];
-    y[i] = apply_act(sum, act);
 }
 
 // ------------------------------------------------------------ convolution --
@@ -746,7 +749,7 @@ hipError_t launch_conv2d_f32(const float *x, const float *w, const float *bias, 
         if (patch_lds(pb) > kLdsMax) pb = 1;
         const bool patch = cb > 1 && K <= KT && patch_lds(pb) <= kLdsMax;
         if (!patch) pb = tiling(false, 2) * group * tiles_c >= 512 ? 2 : 1;
-        if (tiling(patch, pb) * group * tiles_c < ((int64_t)1 << 30)) {
+        if (tiling(patch, pb) * group * tiles_c <= kGridMax) {
             const int64_t lds = patch ? patch_lds(pb) : 0;
             const int64_t grid = group * tiles_c * (patch ? std::min<int64_t>(a.tiles, walk(lds)) : a.tiles);
             auto go = [&](auto cbv, auto pbv) -> hipError_t {
@@ -769,7 +772,7 @@ hipError_t launch_conv2d_f32(const float *x, const float *w, const float *bias, 
             return cb == 1 ? by_pb(One{}) : cb == 2 ? by_pb(Two{}) : by_pb(std::integral_constant<int, 4>{});
         }
     }
-    hipLaunchKernelGGL(k_conv2d_f32, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, x, w, bias, y, C, H, W,
+    hipLaunchKernelGGL(k_conv2d_f32, dim3((unsigned)std::min((total + 255) / 256, kGridMax)), dim3(256), 0, s, x, w, bias, y, C, H, W,
                        Cout, KH, KW, sh, sw, ph, pw, dh, dw, group, OH, OW, act, total);
     return hipGetLastError();
 }

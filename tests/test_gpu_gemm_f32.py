@@ -83,3 +83,17 @@ def test_conv_f32_is_the_fma_chain(dev, case, weight):
                         (st, st), (pd, pd), (dl, dl), group, act=capi.ACT_RELU)
     ref = oracle.conv2d(x, wt, b, strides=(st, st), pads=(pd, pd), dilations=(dl, dl), group=group, act=oracle.ACT_RELU)
     assert np.array_equal(y.cpu().numpy(), ref, equal_nan=True)
+
+
+def test_conv_f32_many_small_images(dev):
+    """More images than one grid dimension has workgroups: every output is written."""
+    n, c, cout = (1 << 24) + 3, 4, 4
+    x = torch.randn(n, c, 1, 1, device=dev, generator=torch.Generator(device=dev).manual_seed(5))
+    wt = synth.normal(1, (cout, c, 1, 1))
+    w = torch.from_numpy(wt).to(dev)
+    y = torch.full((n, cout, 1, 1), np.nan, device=dev)
+    capi._check(capi.lib().lcml_fp8_conv2d_f32(x.data_ptr(), w.data_ptr(), None, y.data_ptr(), n, c, 1, 1, cout, 1, 1, 1, 1,
+                                               0, 0, 1, 1, 1, 1, 1, capi.ACT_NONE, capi._stream()))
+    assert not bool(torch.isnan(y).any())
+    for at in (slice(0, 999), slice((1 << 24) - 500, n)):
+        assert np.array_equal(y[at].cpu().numpy(), oracle.conv2d(x[at].cpu().numpy(), wt, np.zeros(cout, np.float32)))
