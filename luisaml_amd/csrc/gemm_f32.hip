@@ -798,26 +798,27 @@ void launch_sgemm_tile(int M, int N, int K, const float *A, int lda, bool a_kc, 
 hipError_t launch_sgemm(int64_t M, int64_t N, int64_t K, const float *A, int64_t lda, int transA, const float *B,
                         int64_t ldb, int transB, const Epilogue &e, hipStream_t s) {
     auto tiles = [&](int64_t t) { return ((M + t - 1) / t) * ((N + t - 1) / t); };
+    // The tile, in units of one 16x16 block's chain (32 cycles per four
+    // k): a workgroup of 64x64 runs four per SIMD, one of 32x32 one, but
+    // no less than the chain's latency (40 cycles).
+    const int64_t t64 = tiles(64), t32 = tiles(32), t16 = tiles(16);
+    const double c64 = 4.0 * (double)((t64 + 255) / 256), c32 = std::max(1.25, 1.5 * (double)((t32 + 255) / 256));
+    const int tb = t16 <= 256 ? 16 : c32 < c64 ? 32 : 64;
     // a tile's loads stay within 32-bit buffer extents: 128 rows of pitch
     constexpr int64_t kPitchMax = (int64_t)1 << 22;
     if (lda < kPitchMax && ldb < kPitchMax && M < ((int64_t)1 << 30) && N < ((int64_t)1 << 30) &&
-        K < ((int64_t)1 << 30) && tiles(64) < ((int64_t)1 << 31)) {
+        K < ((int64_t)1 << 30) && tiles(tb) <= kGridMax) {
         // 16-byte loads: pointer, pitch and the extent they run along (K, or
         // the operand's rows) whole vectors
         auto whole = [](const float *p, int64_t ld, int64_t extent) {
             return (reinterpret_cast<uintptr_t>(p) & 15) == 0 && ld % 4 == 0 && extent % 4 == 0;
         };
         const bool vec = whole(A, lda, transA ? M : K) && whole(B, ldb, transB ? K : N);
-        // The tile, in units of one 16x16 block's chain (32 cycles per four
-        // k): a workgroup of 64x64 runs four per SIMD, one of 32x32 one, but
-        // no less than the chain's latency (40 cycles).
-        const int64_t t64 = tiles(64), t32 = tiles(32), t16 = tiles(16);
-        const double c64 = 4.0 * (double)((t64 + 255) / 256), c32 = std::max(1.25, 1.5 * (double)((t32 + 255) / 256));
 #define LCML_SGEMM(TB)                                                                                            \
     launch_sgemm_tile<TB>((int)M, (int)N, (int)K, A, (int)lda, !transA, B, (int)ldb, transB != 0, vec, e, s)
-        if (t16 <= 256)
+        if (tb == 16)
             LCML_SGEMM(16);
-        else if (c32 < c64)
+        else if (tb == 32)
             LCML_SGEMM(32);
         else
             LCML_SGEMM(64);

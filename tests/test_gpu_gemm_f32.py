@@ -58,6 +58,19 @@ def test_sgemm_infinities_stay_in_their_row(dev, tb):
     assert np.array_equal(sgemm(dev, a, b, 0, tb, bias, 0, 0), ref, equal_nan=True)
 
 
+def test_sgemm_more_tiles_than_a_grid(dev):
+    """One row by 2^29 columns: more tiles than one grid dimension has workgroups."""
+    N, K = (1 << 29) + 5, 25
+    b = torch.empty((N, K), device=dev).normal_(generator=torch.Generator(device=dev).manual_seed(3))
+    a = synth.normal(1, (1, K))
+    da, y = torch.from_numpy(a).to(dev), torch.full((1, N), np.nan, device=dev)
+    capi._check(capi.lib().lcml_fp8_sgemm(1, N, K, da.data_ptr(), K, 0, b.data_ptr(), K, 1, 1.0, None, 0, 0, 0, 0.0,
+                                          capi.ACT_NONE, y.data_ptr(), capi.DTYPE_FLOAT, N, capi._stream()))
+    assert not bool(torch.isnan(y).any())
+    for at in (slice(0, 999), slice((1 << 29) - 500, N)):
+        assert np.array_equal(y[:, at].cpu().numpy(), oracle.gemm(a, b[at].cpu().numpy(), transB=1))
+
+
 # n, c, h, w, cout, kh, kw, stride, pad, dilation, group: one, two and four
 # 16-channel blocks with and without a remainder, one and two pixels per lane
 # (few and many pixels, odd planes), K of one part (160), just over it and
