@@ -268,9 +268,11 @@ bool w8a32_mfma_wins(int64_t M, int64_t N, int64_t K, int64_t lda) {
     const int64_t panels = pad_to(N, kPanelCols) / 64;
     const double w = (double)panels * (double)M;
     if (w <= 1024 && w * (double)K <= (w <= 512 ? 1.1e6 : 3e5)) return false;
-    // a row group's activations, a panel, the grid at 16 rows per workgroup
+    // a row group's activations, a panel, and the grid at 16 rows per
+    // workgroup of 512: a launch of 2^32 work items or more runs with that
+    // number modulo 2^32 and reports no error
     return (32 * lda + K) * 4 < ((int64_t)1 << 31) && pad_to(K, kPackK) * 64 < ((int64_t)1 << 31) &&
-           M < ((int64_t)1 << 31) - 64 && panels * ((M + 15) / 16) < ((int64_t)1 << 31);
+           M < ((int64_t)1 << 31) - 64 && panels * ((M + 15) / 16) < ((int64_t)1 << 23);
 }
 
 hipError_t launch_gemm_w8a32(int64_t M, int64_t N, int64_t K, const float *a, int64_t lda, const uint8_t *bp,

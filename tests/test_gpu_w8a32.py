@@ -81,3 +81,13 @@ def test_w8a32_infinities_and_nan(dev, M, N):
     assert np.array_equal(np.sign(y[np.isinf(y)]), np.sign(ref[np.isinf(ref)]))
     fin = np.isfinite(ref).all(1)
     check(y[fin], a[fin], qw, sw, bias)
+
+
+def test_w8a32_more_row_groups_than_a_grid(dev):
+    """One column, 2^27 rows: more row groups than one grid dimension has workgroups."""
+    M = (1 << 27) + 16
+    a = torch.empty((M, 1), device=dev).normal_(generator=torch.Generator(device=dev).manual_seed(3))
+    qw, sw = np.array([[0x42]], np.uint8), np.array([0.5], np.float32)
+    y = torch.full((M, 1), np.nan, device=dev)
+    capi.gemm_w8a32(a, capi.pack_weight(torch.from_numpy(qw).to(dev), True), torch.from_numpy(sw).to(dev), 1, 1, out=y)
+    assert torch.equal(y, a * float(oracle.e4m3_to_float(qw)[0, 0]) * 0.5)
