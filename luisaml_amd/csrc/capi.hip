@@ -231,14 +231,16 @@ AutoChoice auto_gemm_choice(int64_t M, int64_t N, int64_t K) {
 int auto_gemm_kernel(int64_t M, int64_t N, int64_t K) { return auto_gemm_choice(M, N, K).kernel; }
 
 // Whether AUTO's dynamically quantised linear of M > 16 rows takes the codes
-// in 16-row blocks and the kernel that reads them: where that one's modelled
-// time is a seventh below the row-major choice's (19 us a unit at K = 4096, 3 us
-// besides; the 128x128 tiles often take that much less than their unit).  N =
-// 12288, K = 4096, with the quantiser: M = 100 31.7 us row-major against 28.1,
-// 256 43.1 against 43.4, 512 66 against 79.
+// in 16-row blocks and the kernel that reads them: where the row-major choice
+// is the small-M kernel, whose sums that kernel's equal bit for bit (the tiles
+// sum K in one chain, and a linear in one call equals its two calls), and its
+// modelled time is a seventh below (19 us a unit at K = 4096, 3 us besides).
+// N = 12288, K = 4096, with the quantiser: M = 100 31.7 us row-major against
+// 28.1.
 bool dynamic_by_rows(int64_t M, int64_t N, int64_t K) {
-    return M > 16 &&
-           lcml::gemm_rows_us(M, N, K) < 0.86 * (auto_gemm_choice(M, N, K).units * 19.0 * (double)K / 4096.0 + 3.0);
+    const AutoChoice c = auto_gemm_choice(M, N, K);
+    return M > 16 && c.kernel == LCML_KERNEL_SKINNY &&
+           lcml::gemm_rows_us(M, N, K) < 0.86 * (c.units * 19.0 * (double)K / 4096.0 + 3.0);
 }
 }  // namespace
 

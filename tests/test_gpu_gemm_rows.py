@@ -78,3 +78,26 @@ def test_rows_partials_strides_and_alignment(dev):
         assert np.array_equal(np.isnan(a), np.isnan(b))
         ok = ~np.isnan(a)
         assert np.allclose(a[ok], b[ok], rtol=1e-4, atol=1e-5 * np.abs(a[ok]).max())
+
+
+# either side of the sizes where the row-major choice turns from the small-M
+# kernel to the tiles, and sizes well inside either
+@pytest.mark.parametrize("M,N,K", [(17, 1000, 1040), (64, 12288, 2048), (100, 4096, 2064), (100, 11008, 4096),
+                                   (160, 11008, 2048), (161, 11008, 2048), (200, 11008, 4096), (512, 4096, 1024),
+                                   (513, 4096, 1024), (600, 4096, 2048), (300, 8192, 1024), (180, 12288, 2048),
+                                   (1100, 2048, 1024), (2100, 1024, 1024)])
+@pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
+def test_one_call_equals_two(dev, M, N, K, out_dtype):
+    """gemm_dynamic is quantize_dynamic followed by gemm bit for bit, whatever
+    kernels either takes, and whether or not x is 16-byte aligned."""
+    g = torch.Generator(device=dev).manual_seed(M + N)
+    buf = torch.empty(M * K + 1, device=dev).normal_(generator=g)
+    x, xm = buf[:M * K].view(M, K), buf[1:].view(M, K)
+    q = torch.empty((N, K), device=dev).normal_(0.0, 0.05, generator=g)
+    bp = capi.pack_weight(capi.quantize(q, torch.full((1,), 2.0 ** -11, device=dev)), True)
+    sw = torch.empty(N, device=dev).uniform_(1e-4, 1e-3, generator=g)
+    kw = dict(c=torch.empty(N, device=dev).normal_(generator=g), act=capi.ACT_GELU_ERF, out_dtype=out_dtype)
+    for v in (x, xm):
+        codes, s = capi.quantize_dynamic(v)
+        two = capi.gemm(codes, s, bp, sw, N, K, **kw)
+        assert torch.equal(capi.gemm_dynamic(v, bp, sw, N, K, **kw), two)
