@@ -9,8 +9,9 @@
 // v_mfma_f32_16x16x32_bf16 give sum_k x_k w_k with fewer roundings than an fma
 // chain over k has (one per 32 products; error against 64 bits at 128 x 11008
 // x 4096 1.1e-7 of the norm, 3.0e-7 with the fma chains).  Three of them take 48 cycles of a
-// SIMD for 8192 multiply-adds; v_fma_f32 takes 512.  (Bits of x below 2^-133,
-// the smallest bf16 value, are dropped.)
+// SIMD for 8192 multiply-adds; v_fma_f32 takes 512.  The activations are
+// split times 2^16, so that bf16's smallest value, 2^-133, holds the last bit of
+// every one, subnormals among them, and the sums are scaled back.
 //
 // What is left is shaped as the small-M FP8 GEMM: a workgroup of 8
 // wavefronts owns 16*MB rows and one 64-column panel; the wavefronts split K
@@ -20,10 +21,12 @@
 // operations and is repeated by every panel's workgroup; beside 12 MFMAs per
 // 16 of them it hides.
 //
-// An activation that is inf or NaN leaves NaN in mid and lo.  The wavefronts
-// test their sums for NaN once, at the end, and if there is one the workgroup
-// runs again with mid = lo = 0 for those activations (SPECIAL): then inf * w
-// is the fma chain's.
+// An activation that is inf, NaN or from 2^112 on leaves NaN in mid and lo.
+// The wavefronts test their sums for NaN and infinities once, at the end, and
+// if there is one the workgroup runs twice again: over the activations below
+// 2^-64 as before, and, adding to those sums, over the others without the
+// factor and with mid = lo = 0 where they are not finite: then inf * w is the
+// fma chain's, and what is small keeps its bits beside it.
 #include <algorithm>
 
 #include "lcml_internal.hpp"
@@ -49,18 +52,29 @@ __device__ inline uint32_t upper2(float a, float b) {
     return __builtin_amdgcn_perm(f32_bits(b), f32_bits(a), 0x07060302u);
 }
 
-template <bool SPECIAL>
+// Which activations a run over K takes, and how.  bf16 ends at 2^-133, fp32 at
+// 2^-149: times 2^16 no bit of an activation is lost.
+enum Run {
+    kAll,    // every one, times 2^16 (NaN in the lower pieces where that is not finite)
+    kSmall,  // those below 2^-64, times 2^16
+    kRest,   // the others as they are, inf and NaN among them
+};
+constexpr float kUp = 0x1p16f, kDown = 0x1p-16f, kSmallMax = 0x1p-64f;
+
+template <Run RUN>
 __device__ inline Split split4(f4 x) {
     float h[4], m[4], l[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        h[i] = bits_f32(f32_bits(x[i]) & 0xffff0000u);
-        const float r = x[i] - h[i];
+        const bool small = fabsf(x[i]) < kSmallMax;
+        const float v = RUN == kAll ? x[i] * kUp : RUN == kSmall ? (small ? x[i] * kUp : 0.0f) : small ? 0.0f : x[i];
+        h[i] = bits_f32(f32_bits(v) & 0xffff0000u);
+        const float r = v - h[i];
         m[i] = bits_f32(f32_bits(r) & 0xffff0000u);
         l[i] = r - m[i];
-        if constexpr (SPECIAL)
-            if (!(fabsf(x[i]) <= 3.4028235e38f)) {
-                h[i] = x[i] != x[i] ? bits_f32(0x7fc00000u) : x[i];  // a NaN's upper half may be an infinity's
+        if constexpr (RUN == kRest)
+            if (!(fabsf(v) <= 3.4028235e38f)) {
+                h[i] = v != v ? bits_f32(0x7fc00000u) : v;  // a NaN's upper half may be an infinity's
                 m[i] = l[i] = 0.0f;
             }
     }
@@ -86,7 +100,7 @@ __device__ inline Split split4(f4 x) {
 // count.  The leading scalar arguments arrive in SGPRs
 // (-amdgpu-kernarg-preload-count).
 template <int MB, int P, int KS, bool VEC>
-__global__ __launch_bounds__(P *KS * 64) void k_gemm_w8a32(const uint8_t *bp, const float *a, int lda, int M, int K,
+__global__ __launch_bounds__(P *KS * 64, P == 2 && VEC ? 4 : 1) void k_gemm_w8a32(const uint8_t *bp, const float *a, int lda, int M, int K,
                                                             int kc, int npanels, int rg, Epilogue e) {
     constexpr int ROWS = 16 * MB, PITCH = 144, PIECE = ROWS * PITCH, BUF = 3 * PIECE;
     constexpr int XL = (ROWS * 16 + 64 * P - 1) / (64 * P);  // float4s of a step per thread
@@ -138,12 +152,12 @@ __global__ __launch_bounds__(P *KS * 64) void k_gemm_w8a32(const uint8_t *bp, co
 #pragma unroll
         for (int j = 0; j < 4; ++j) w[j] = __builtin_amdgcn_raw_buffer_load_b128(br, (int)(o + j * 256), 0, 0);
     };
-    auto put_x = [&](int b, auto special) {
+    auto put_x = [&](int b, auto which) {
 #pragma unroll
         for (int u = 0; u < XL; ++u) {
             if (ROWS * 16 % (64 * P) != 0 && (pt >> 4) + 4 * P * u >= ROWS) continue;
             uint8_t *to = buf + b * BUF + ((pt >> 4) + 4 * P * u) * PITCH + (pt & 15) * 8;
-            const Split s = split4<decltype(special)::value>(x[u]);
+            const Split s = split4<decltype(which)::value>(x[u]);
             *reinterpret_cast<u2 *>(to) = s.hi;
             *reinterpret_cast<u2 *>(to + PIECE) = s.mid;
             *reinterpret_cast<u2 *>(to + 2 * PIECE) = s.lo;
@@ -177,14 +191,18 @@ __global__ __launch_bounds__(P *KS * 64) void k_gemm_w8a32(const uint8_t *bp, co
             }
         }
     };
-    auto run = [&](auto special) {
+    auto run = [&](auto which) {
+        constexpr Run RUN = decltype(which)::value;
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) acc[mb][j] = low[mb][j] = v4f{0.f, 0.f, 0.f, 0.f};
+            for (int j = 0; j < 4; ++j) {
+                if (RUN != kRest) acc[mb][j] = v4f{0.f, 0.f, 0.f, 0.f};  // kRest adds to kSmall's sums
+                low[mb][j] = v4f{0.f, 0.f, 0.f, 0.f};
+            }
         load_x(s_begin);
         load_w(w[0], s_begin);
-        put_x(0, special);
+        put_x(0, which);
         load_x(s_begin + 1);
         __syncthreads();
         for (int i0 = 0; i0 < steps; i0 += 2) {
@@ -193,7 +211,7 @@ __global__ __launch_bounds__(P *KS * 64) void k_gemm_w8a32(const uint8_t *bp, co
                 const int i = i0 + d;
                 if (i >= steps) break;
                 load_w(w[1 - d], s_begin + i + 1);
-                put_x(1 - d, special);
+                put_x(1 - d, which);
                 load_x(s_begin + i + 2);
                 __builtin_amdgcn_sched_barrier(0);
                 compute(w[d], d);
@@ -203,9 +221,12 @@ __global__ __launch_bounds__(P *KS * 64) void k_gemm_w8a32(const uint8_t *bp, co
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) acc[mb][j] += low[mb][j];
+            for (int j = 0; j < 4; ++j) {
+                acc[mb][j] += low[mb][j];
+                if (RUN != kRest) acc[mb][j] *= kDown;
+            }
     };
-    run(std::false_type{});
+    run(std::integral_constant<Run, kAll>{});
     float nan = 0.0f;
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
@@ -213,8 +234,11 @@ __global__ __launch_bounds__(P *KS * 64) void k_gemm_w8a32(const uint8_t *bp, co
         for (int j = 0; j < 4; ++j)
 #pragma unroll
             for (int r = 0; r < 4; ++r) nan = fmaf(acc[mb][j][r], 0.0f, nan);
-    // (an infinite sum, 0 * inf, counts too: the second run gives it again)
-    if (__builtin_expect(__syncthreads_or(nan != nan), 0)) run(std::true_type{});
+    // (an infinite sum, 0 * inf, counts too: the factor may have made it)
+    if (__builtin_expect(__syncthreads_or(nan != nan), 0)) {
+        run(std::integral_constant<Run, kSmall>{});
+        run(std::integral_constant<Run, kRest>{});
+    }
 
     // the parts' sums through LDS, [wave][block][register][lane]: register r
     // of lane l of block j is row (l/16)*4 + r, column l%16

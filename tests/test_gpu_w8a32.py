@@ -50,19 +50,46 @@ def test_w8a32_against_64_bits(dev, M, N, K, pad, shift):
     check(run(dev, a, qw, sw, bias, pad, shift).cpu().numpy(), a, qw, sw, bias)
 
 
-@pytest.mark.parametrize("scale", [1e-38, 1e-30, 1e30])
-def test_w8a32_ends_of_the_range(dev, scale):
-    """Subnormal pieces, and values near the largest: the bound plus what the
-    smallest bf16 value (2^-133) drops of each activation."""
-    M, N, K = 40, 2048, 256
+def check_unscaled(y, a, B):
+    """check() for unit scales; at most 8 parts' sums, their sum and the result
+    are each rounded to a multiple of 2^-149."""
+    K = a.shape[1]
+    ref = a.astype(np.float64) @ B.T
+    bound = (K + 3) * 2.0 ** -24 * (np.abs(a).astype(np.float64) @ np.abs(B).T) + 17 * 2.0 ** -150
+    assert np.all(np.abs(y.astype(np.float64) - ref) <= bound)
+
+
+@pytest.mark.parametrize("scale", [1e-43, 1e-40, 1e-38, 1e-36, 1e-33, 1e-30, 1e30, 1e34])
+@pytest.mark.parametrize("M,N", [(40, 2048), (40, 11008), (128, 11008)])
+def test_w8a32_ends_of_the_range(dev, M, N, scale):
+    """Subnormal activations and pieces, and values near the largest: the same bound."""
+    K = 256
     a = (synth.normal(1, (M, K)) * scale).astype(np.float32)
     qw, sw = weights(N, K, 2)
-    sw = np.ones_like(sw)
+    y = run(dev, a, qw, np.ones_like(sw), np.zeros(N, np.float32)).cpu().numpy()
+    check_unscaled(y, a, oracle.e4m3_to_float(qw).astype(np.float64))
+
+
+@pytest.mark.parametrize("big", [2.0 ** 111, 2.0 ** 112, 2.0 ** 113, 2.0 ** 118, np.inf])
+def test_w8a32_small_beside_large(dev, big):
+    """Activations at the ends of the range in one workgroup, in other rows and
+    in one row whose large values meet zero weights: the small ones keep their
+    bits, and an infinity's row has none to keep."""
+    M, N, K = 40, 2048, 256
+    a = (synth.normal(1, (M, K)) * np.exp(synth.normal(2, (M, K), std=20.0)) * 1e-38).astype(np.float32)
+    qw, _ = weights(N, K, 2)
+    qw[:N // 2, 7] = 0
+    a[3, 7] = a[30, 7] = np.float32(big)
+    a[5, 9] = np.float32(big)
+    y = run(dev, a, qw, np.ones(N, np.float32), np.zeros(N, np.float32)).cpu().numpy()
     B = oracle.e4m3_to_float(qw).astype(np.float64)
-    y = run(dev, a, qw, sw, np.zeros(N, np.float32)).cpu().numpy().astype(np.float64)
-    ref = a.astype(np.float64) @ B.T
-    bound = (K + 3) * 2.0 ** -24 * (np.abs(a).astype(np.float64) @ np.abs(B).T) + 2.0 ** -133 * np.abs(B).sum(1)
-    assert np.all(np.abs(y - ref) <= bound)
+    if np.isinf(big):
+        ref = oracle.gemm(a, oracle.e4m3_to_float(qw), transB=1)
+        for r in (3, 5, 30):
+            assert np.array_equal(np.isnan(y[r]), np.isnan(ref[r])) and not np.isfinite(y[r]).any()
+        fin = [r for r in range(M) if r not in (3, 5, 30)]
+        y, a = y[fin], a[fin]
+    check_unscaled(y, a, B)
 
 
 @pytest.mark.parametrize("M,N", [(40, 2048), (40, 11008), (128, 11008)])
