@@ -76,7 +76,7 @@ def test_w8a32_small_beside_large(dev, big):
     in one row whose large values meet zero weights: the small ones keep their
     bits, and an infinity's row has none to keep."""
     M, N, K = 40, 2048, 256
-    a = (synth.normal(1, (M, K)) * np.exp(synth.normal(2, (M, K), std=20.0)) * 1e-38).astype(np.float32)
+    a = (synth.normal(1, (M, K)) * np.float32(1e-38)).astype(np.float32)
     qw, _ = weights(N, K, 2)
     qw[:N // 2, 7] = 0
     a[3, 7] = a[30, 7] = np.float32(big)
