@@ -115,8 +115,9 @@ int lcml_fp8_quantize(const float *x, uint8_t *y, int64_t outer, int64_t axis_le
     if (int rc = check_view(outer, axis_len, inner, "lcml_fp8_quantize")) return rc;
     if (outer * axis_len * inner == 0) return LCML_OK;
     if (!x || !y || !y_scale) return fail(LCML_ERR_INVALID_ARG, "lcml_fp8_quantize: NULL pointer");
-    return hip_status(lcml::launch_quantize(x, y, outer, axis_len, inner, y_scale, (hipStream_t)stream),
-                      "lcml_fp8_quantize");
+    const char *label = nullptr;
+    const hipError_t err = lcml::launch_quantize(x, y, outer, axis_len, inner, y_scale, (hipStream_t)stream, &label);
+    return hip_status(err, "lcml_fp8_quantize", label);
 }
 
 int lcml_fp8_dequantize(const uint8_t *x, float *y, int64_t outer, int64_t axis_len, int64_t inner,
@@ -124,8 +125,9 @@ int lcml_fp8_dequantize(const uint8_t *x, float *y, int64_t outer, int64_t axis_
     if (int rc = check_view(outer, axis_len, inner, "lcml_fp8_dequantize")) return rc;
     if (outer * axis_len * inner == 0) return LCML_OK;
     if (!x || !y || !x_scale) return fail(LCML_ERR_INVALID_ARG, "lcml_fp8_dequantize: NULL pointer");
-    return hip_status(lcml::launch_dequantize(x, y, outer, axis_len, inner, x_scale, (hipStream_t)stream),
-                      "lcml_fp8_dequantize");
+    const char *label = nullptr;
+    const hipError_t err = lcml::launch_dequantize(x, y, outer, axis_len, inner, x_scale, (hipStream_t)stream, &label);
+    return hip_status(err, "lcml_fp8_dequantize", label);
 }
 
 int lcml_fp8_quantize_dynamic(const float *x, uint8_t *y, int64_t n, float *scale_out, void *workspace,

@@ -11,10 +11,11 @@
 
 namespace lcml {
 
+// (*kernel: the chosen kernel's name in the kernel trace)
 hipError_t launch_quantize(const float *x, uint8_t *y, int64_t outer, int64_t axis_len,
-                           int64_t inner, const float *scale, hipStream_t s);
+                           int64_t inner, const float *scale, hipStream_t s, const char **kernel);
 hipError_t launch_dequantize(const uint8_t *x, float *y, int64_t outer, int64_t axis_len,
-                             int64_t inner, const float *scale, hipStream_t s);
+                             int64_t inner, const float *scale, hipStream_t s, const char **kernel);
 // amax into a zero-initialised uint word (atomic max on fp32 bits)
 hipError_t launch_amax(const float *x, int64_t n, uint32_t *amax_bits, hipStream_t s);
 // partial maxima (at most kMaxAmaxPartials words at part); *npart = count

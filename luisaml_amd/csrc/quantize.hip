@@ -140,16 +140,17 @@ __global__ __launch_bounds__(kThreads) void k_quantize_cols(const float *__restr
         run(std::false_type{});
 }
 
-// Any other axis: the first element's place by one 32-bit division (n below
-// 2^32), the others by counting; the reciprocal changes where a group
-// crosses into the next scale's run.
+// Any other axis: the first element's place by a division in I (uint32_t for n
+// below 2^32, else uint64_t), the others by counting; the reciprocal changes
+// where a group crosses into the next scale's run.
+template <class I>
 __global__ __launch_bounds__(kThreads) void k_quantize_axis(const float *__restrict__ x, uint8_t *__restrict__ y,
-                                                            int64_t n, uint32_t axis_len, uint32_t inner, int wraps,
+                                                            int64_t n, I axis_len, I inner, int wraps,
                                                             const float *__restrict__ scale) {
     const f4 *x4 = reinterpret_cast<const f4 *>(x);
     uint32_t *y4 = reinterpret_cast<uint32_t *>(y);
     const int64_t n4 = n >> 2, stride = (int64_t)gridDim.x * kThreads * kUc;
-    auto place = [&](uint32_t e, uint32_t &a, uint32_t &rem) {
+    auto place = [&](I e, I &a, I &rem) {
         a = e / inner;
         rem = e - a * inner;
         if (wraps) a %= axis_len;
@@ -157,12 +158,12 @@ __global__ __launch_bounds__(kThreads) void k_quantize_axis(const float *__restr
     for (int64_t i0 = (int64_t)blockIdx.x * kThreads * kUc + threadIdx.x; i0 < n4; i0 += stride) {
         f4 v[kUc];
         float s[kUc];
-        uint32_t a[kUc], rem[kUc];
+        I a[kUc], rem[kUc];
 #pragma unroll
         for (int u = 0; u < kUc; ++u) {
             const int64_t i = i0 + (int64_t)u * kThreads;
             v[u] = i < n4 ? __builtin_nontemporal_load(x4 + i) : f4{0.f, 0.f, 0.f, 0.f};
-            place(i < n4 ? (uint32_t)i * 4 : 0u, a[u], rem[u]);
+            place(i < n4 ? (I)i * 4 : (I)0, a[u], rem[u]);
             s[u] = scale[a[u]];
         }
 #pragma unroll
@@ -183,8 +184,8 @@ __global__ __launch_bounds__(kThreads) void k_quantize_axis(const float *__restr
         }
     }
     if (blockIdx.x == 0 && threadIdx.x < (n & 3)) {
-        uint32_t at, rt;
-        place((uint32_t)n4 * 4 + threadIdx.x, at, rt);
+        I at, rt;
+        place((I)n4 * 4 + threadIdx.x, at, rt);
         quantize_tail(x, y, n4 * 4 + threadIdx.x, scale[at]);
     }
 }
@@ -280,25 +281,27 @@ __global__ __launch_bounds__(kThreads) void k_dequantize_cols(const uint8_t *__r
     }
 }
 
+template <class I>
 __global__ __launch_bounds__(kThreads) void k_dequantize_axis(const uint8_t *__restrict__ q, float *__restrict__ y,
-                                                              int64_t n, uint32_t axis_len, uint32_t inner, int wraps,
+                                                              int64_t n, I axis_len, I inner, int wraps,
                                                               const float *__restrict__ scale) {
     const uint32_t *q4 = reinterpret_cast<const uint32_t *>(q);
     f4 *y4 = reinterpret_cast<f4 *>(y);
     const int64_t n4 = n >> 2, stride = (int64_t)gridDim.x * kThreads * kUc;
-    auto place = [&](uint32_t e, uint32_t &a, uint32_t &rem) {
+    auto place = [&](I e, I &a, I &rem) {
         a = e / inner;
         rem = e - a * inner;
         if (wraps) a %= axis_len;
     };
     for (int64_t i0 = (int64_t)blockIdx.x * kThreads * kUc + threadIdx.x; i0 < n4; i0 += stride) {
-        uint32_t w[kUc], a[kUc], rem[kUc];
+        uint32_t w[kUc];
+        I a[kUc], rem[kUc];
         float s[kUc];
 #pragma unroll
         for (int u = 0; u < kUc; ++u) {
             const int64_t i = i0 + (int64_t)u * kThreads;
             w[u] = i < n4 ? __builtin_nontemporal_load(q4 + i) : 0u;
-            place(i < n4 ? (uint32_t)i * 4 : 0u, a[u], rem[u]);
+            place(i < n4 ? (I)i * 4 : (I)0, a[u], rem[u]);
             s[u] = scale[a[u]];
         }
 #pragma unroll
@@ -321,8 +324,8 @@ __global__ __launch_bounds__(kThreads) void k_dequantize_axis(const uint8_t *__r
         }
     }
     if (blockIdx.x == 0 && threadIdx.x < (n & 3)) {
-        uint32_t at, rt;
-        place((uint32_t)n4 * 4 + threadIdx.x, at, rt);
+        I at, rt;
+        place((I)n4 * 4 + threadIdx.x, at, rt);
         dequantize_tail(q, y, n4 * 4 + threadIdx.x, scale[at]);
     }
 }
@@ -562,7 +565,8 @@ ColsPlan plan_cols(int64_t n4, int64_t axis_len) {
 }  // namespace
 
 hipError_t launch_quantize(const float *x, uint8_t *y, int64_t outer, int64_t axis_len,
-                           int64_t inner, const float *scale, hipStream_t s) {
+                           int64_t inner, const float *scale, hipStream_t s, const char **kernel) {
+    *kernel = "quantize_vec";
     const int64_t n = outer * axis_len * inner;
     if (n == 0) return hipSuccess;
     const bool vec = aligned16(x) && aligned4(y);
@@ -570,13 +574,20 @@ hipError_t launch_quantize(const float *x, uint8_t *y, int64_t outer, int64_t ax
         hipLaunchKernelGGL(k_quantize_vec<false>, dim3(grid_vec(n / 4, kU)), dim3(kThreads), 0, s, x, y, n, scale,
                            nullptr, 0, nullptr);
     } else if (vec && inner == 1 && axis_len < ((int64_t)1 << 30)) {
+        *kernel = "quantize_cols";
         const ColsPlan p = plan_cols(n / 4, axis_len);
         hipLaunchKernelGGL(k_quantize_cols, dim3(p.grid), dim3(kThreads), 0, s, x, y, n, p.Lq, p.T, (uint32_t)axis_len,
                            scale);
     } else if (vec && n < ((int64_t)1 << 32)) {
-        hipLaunchKernelGGL(k_quantize_axis, dim3(grid_vec(n / 4, kUc)), dim3(kThreads), 0, s, x, y, n,
+        *kernel = "quantize_axis";
+        hipLaunchKernelGGL(k_quantize_axis<uint32_t>, dim3(grid_vec(n / 4, kUc)), dim3(kThreads), 0, s, x, y, n,
                            (uint32_t)axis_len, (uint32_t)inner, outer > 1 ? 1 : 0, scale);
+    } else if (vec) {
+        *kernel = "quantize_axis";
+        hipLaunchKernelGGL(k_quantize_axis<uint64_t>, dim3(grid_vec(n / 4, kUc)), dim3(kThreads), 0, s, x, y, n,
+                           (uint64_t)axis_len, (uint64_t)inner, outer > 1 ? 1 : 0, scale);
     } else {
+        *kernel = "quantize_scalar";
         hipLaunchKernelGGL(k_quantize_scalar<false>, dim3(grid_for(n)), dim3(kThreads), 0, s, x, y, n,
                            axis_len, inner, scale, nullptr, 0, nullptr);
     }
@@ -584,20 +595,28 @@ hipError_t launch_quantize(const float *x, uint8_t *y, int64_t outer, int64_t ax
 }
 
 hipError_t launch_dequantize(const uint8_t *x, float *y, int64_t outer, int64_t axis_len,
-                             int64_t inner, const float *scale, hipStream_t s) {
+                             int64_t inner, const float *scale, hipStream_t s, const char **kernel) {
+    *kernel = "dequantize_vec";
     const int64_t n = outer * axis_len * inner;
     if (n == 0) return hipSuccess;
     const bool vec = aligned4(x) && aligned16(y);
     if (vec && axis_len == 1) {
         hipLaunchKernelGGL(k_dequantize_vec, dim3(grid_vec(n / 4, kUd)), dim3(kThreads), 0, s, x, y, n, scale);
     } else if (vec && inner == 1 && axis_len < ((int64_t)1 << 30)) {
+        *kernel = "dequantize_cols";
         const ColsPlan p = plan_cols(n / 4, axis_len);
         hipLaunchKernelGGL(k_dequantize_cols, dim3(p.grid), dim3(kThreads), 0, s, x, y, n, p.Lq, p.T,
                            (uint32_t)axis_len, scale);
     } else if (vec && n < ((int64_t)1 << 32)) {
-        hipLaunchKernelGGL(k_dequantize_axis, dim3(grid_vec(n / 4, kUc)), dim3(kThreads), 0, s, x, y, n,
+        *kernel = "dequantize_axis";
+        hipLaunchKernelGGL(k_dequantize_axis<uint32_t>, dim3(grid_vec(n / 4, kUc)), dim3(kThreads), 0, s, x, y, n,
                            (uint32_t)axis_len, (uint32_t)inner, outer > 1 ? 1 : 0, scale);
+    } else if (vec) {
+        *kernel = "dequantize_axis";
+        hipLaunchKernelGGL(k_dequantize_axis<uint64_t>, dim3(grid_vec(n / 4, kUc)), dim3(kThreads), 0, s, x, y, n,
+                           (uint64_t)axis_len, (uint64_t)inner, outer > 1 ? 1 : 0, scale);
     } else {
+        *kernel = "dequantize_scalar";
         hipLaunchKernelGGL(k_dequantize_scalar, dim3(grid_for(n)), dim3(kThreads), 0, s, x, y, n, axis_len, inner,
                            scale);
     }

@@ -44,6 +44,27 @@ def test_per_axis(dev, shape, axis, shift):
     assert np.array_equal(back.cpu().numpy(), oracle.dequantize(ref, s, axis=axis), equal_nan=True)
 
 
+@pytest.mark.parametrize("shape", [(1 << 10, (1 << 12) + 1, 1 << 10), (1 << 16, (1 << 16) + 1, 1), (3, 21, 68191747)])
+def test_per_axis_beyond_32_bits(dev, shape):
+    """2^32 elements and more, with an inner run and without, whole vectors and not."""
+    x = torch.empty(shape, device=dev).normal_(generator=torch.Generator(device=dev).manual_seed(1))
+    s = np.abs(synth.normal(1, (shape[1],), std=0.05)) + np.float32(1e-4)
+    ds = torch.from_numpy(s).to(dev)
+    capi.kernel_trace()
+    q = capi.quantize(x, ds, axis=1)
+    # first, last, and either side of element 2^32
+    inner, n = shape[2], x.numel()
+    xf, qf = x.view(-1), q.view(-1)
+    at = torch.cat([torch.arange(0, 5000), torch.arange((1 << 32) - 5000, min(n, (1 << 32) + 5000)), torch.arange(n - 5000, n)])
+    ref = oracle.quantize(xf[at.to(dev)].cpu().numpy(), s[(at // inner % shape[1]).numpy()], axis=0)
+    assert np.array_equal(qf[at.to(dev)].cpu().numpy(), ref)
+    capi.dequantize(q, ds, axis=1, out=x)
+    back = oracle.dequantize(ref, s[(at // inner % shape[1]).numpy()], axis=0)
+    assert np.array_equal(xf[at.to(dev)].cpu().numpy(), back)
+    kind = "cols" if inner == 1 else "axis"
+    assert capi.kernel_trace() == ["quantize_" + kind, "dequantize_" + kind]
+
+
 @pytest.mark.parametrize("n", [1, 3, 4, 5, 4097, 16387, 65533, 65537, 262147, 2097155, 9000001])
 @pytest.mark.parametrize("shift", [0, 1])
 def test_dynamic_odd_sizes(dev, n, shift):
