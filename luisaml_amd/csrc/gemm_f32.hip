@@ -254,28 +254,28 @@ __global__ __launch_bounds__(256) void k_conv2d_f32(const float *__restrict__ x,
                                                     int H, int W, int Cout, int KH, int KW, int sh, int sw, int ph,
                                                     int pw, int dh, int dw, int group, int OH, int OW, int act,
                                                     int64_t total) {
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
-        const int ow = (int)(i % OW);
-        const int oh = (int)((i / OW) % OH);
-        const int co = (int)((i / ((int64_t)OW * OH)) % Cout);
-        const int64_t n = i / ((int64_t)OW * OH * Cout);
-        const int cg = C / group, mg = Cout / group, g = co / mg;
-        const float *xn = x + (n * C + (int64_t)g * cg) * H * W;
-        const float *wc = w + (int64_t)co * cg * KH * KW;
-        float sum = 0.0f;
-        for (int kh = 0; kh < KH; ++kh) {
-            const int ih = oh * sh + kh * dh - ph;
-            if ((unsigned)ih >= (unsigned)H) continue;
-            for (int kw = 0; kw < KW; ++kw) {
-                const int iw = ow * sw + kw * dw - pw;
-                if ((unsigned)iw >= (unsigned)W) continue;
-                for (int c = 0; c < cg; ++c)
-                    sum = fmaf(xn[((int64_t)c * H + ih) * W + iw], wc[((int64_t)c * KH + kh) * KW + kw], sum);
-            }
+    const int64_t i = ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * 256 + threadIdx.x;
+    if (i >= total) return;
+    const int ow = (int)(i % OW);
+    const int oh = (int)((i / OW) % OH);
+    const int co = (int)((i / ((int64_t)OW * OH)) % Cout);
+    const int64_t n = i / ((int64_t)OW * OH * Cout);
+    const int cg = C / group, mg = Cout / group, g = co / mg;
+    const float *xn = x + (n * C + (int64_t)g * cg) * H * W;
+    const float *wc = w + (int64_t)co * cg * KH * KW;
+    float sum = 0.0f;
+    for (int kh = 0; kh < KH; ++kh) {
+        const int ih = oh * sh + kh * dh - ph;
+        if ((unsigned)ih >= (unsigned)H) continue;
+        for (int kw = 0; kw < KW; ++kw) {
+            const int iw = ow * sw + kw * dw - pw;
+            if ((unsigned)iw >= (unsigned)W) continue;
+            for (int c = 0; c < cg; ++c)
+                sum = fmaf(xn[((int64_t)c * H + ih) * W + iw], wc[((int64_t)c * KH + kh) * KW + kw], sum);
         }
-        if (bias) sum += bias[co];
-        y[i] = apply_act(sum, act);
     }
+    if (bias) sum += bias[co];
+    y[i] = apply_act(sum, act);
 }
 
 // ------------------------------------------------------------ convolution --
@@ -772,7 +772,9 @@ hipError_t launch_conv2d_f32(const float *x, const float *w, const float *bias, 
             return cb == 1 ? by_pb(One{}) : cb == 2 ? by_pb(Two{}) : by_pb(std::integral_constant<int, 4>{});
         }
     }
-    hipLaunchKernelGGL(k_conv2d_f32, dim3((unsigned)std::min((total + 255) / 256, kGridMax)), dim3(256), 0, s, x, w, bias, y, C, H, W,
+    // (a loop over the outputs cost the small planes 10 %)
+    const int64_t wgs = (total + 255) / 256, gx = std::min(wgs, kGridMax);
+    hipLaunchKernelGGL(k_conv2d_f32, dim3((unsigned)gx, (unsigned)((wgs + gx - 1) / gx)), dim3(256), 0, s, x, w, bias, y, C, H, W,
                        Cout, KH, KW, sh, sw, ph, pw, dh, dw, group, OH, OW, act, total);
     return hipGetLastError();
 }

@@ -110,3 +110,17 @@ def test_conv_f32_many_small_images(dev):
     assert not bool(torch.isnan(y).any())
     for at in (slice(0, 999), slice((1 << 24) - 500, n)):
         assert np.array_equal(y[at].cpu().numpy(), oracle.conv2d(x[at].cpu().numpy(), wt, np.zeros(cout, np.float32)))
+
+
+def test_conv_f32_more_outputs_than_a_grid(dev):
+    """2^32 outputs and more of the direct kernel (fewer than four channels a group)."""
+    n, cout = (1 << 31) // 3 + 7, 6
+    x = torch.empty((n, 3, 1, 1), device=dev).normal_(generator=torch.Generator(device=dev).manual_seed(6))
+    wt = synth.normal(2, (cout, 1, 1, 1))
+    w = torch.from_numpy(wt).to(dev)
+    y = torch.full((n, cout, 1, 1), np.nan, device=dev)
+    capi._check(capi.lib().lcml_fp8_conv2d_f32(x.data_ptr(), w.data_ptr(), None, y.data_ptr(), n, 3, 1, 1, cout, 1, 1, 1, 1,
+                                               0, 0, 1, 1, 3, 1, 1, capi.ACT_NONE, capi._stream()))
+    assert y.numel() > 1 << 32 and not bool(torch.isnan(y.view(-1)[-1000:]).any())
+    for at in (slice(0, 999), slice((1 << 32) // cout - 500, (1 << 32) // cout + 7), slice(n - 500, n)):
+        assert np.array_equal(y[at].cpu().numpy(), oracle.conv2d(x[at].cpu().numpy(), wt, np.zeros(cout, np.float32), group=3))
