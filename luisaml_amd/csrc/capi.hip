@@ -673,10 +673,11 @@ int lcml_fp8_conv2d_f32(const float *x, const float *w, const float *bias, float
     if (n == 0) return LCML_OK;
     if (!x || !w || !y) return fail(LCML_ERR_INVALID_ARG, "%s: NULL pointer", fn);
     if (n * cout * oh * ow >= (int64_t)1 << 40) return fail(LCML_ERR_UNSUPPORTED, "%s: output too large", fn);
-    return hip_status(lcml::launch_conv2d_f32(x, w, bias, y, n, (int)c, (int)h, (int)wd, (int)cout, (int)kh, (int)kw,
-                                              (int)stride_h, (int)stride_w, (int)pad_h, (int)pad_w, (int)dil_h,
-                                              (int)dil_w, (int)group, (int)oh, (int)ow, act, (hipStream_t)stream),
-                      fn);
+    const char *label = nullptr;
+    const hipError_t err = lcml::launch_conv2d_f32(
+        x, w, bias, y, n, (int)c, (int)h, (int)wd, (int)cout, (int)kh, (int)kw, (int)stride_h, (int)stride_w,
+        (int)pad_h, (int)pad_w, (int)dil_h, (int)dil_w, (int)group, (int)oh, (int)ow, act, (hipStream_t)stream, &label);
+    return hip_status(err, fn, label);
 }
 
 int lcml_fp8_sgemm(int64_t M, int64_t N, int64_t K, const float *a, int64_t lda, int trans_a, const float *b,

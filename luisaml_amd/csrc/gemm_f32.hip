@@ -12,6 +12,7 @@
 // for each of four exponent ranges, subnormals among them), at twice the
 // rate of v_fma_f32 and without a register operand per product and lane.
 #include <algorithm>
+#include <cmath>
 
 #include "lcml_internal.hpp"
 
@@ -247,8 +248,8 @@ __global__ __launch_bounds__(256) void k_activation(const float *__restrict__ x,
 // group's input channels; conv.cpp:143-192, whose 4-wide partial sums differ
 // from this chain only in fp32 rounding), begin pads only (conv.cpp:121),
 // dilation, groups, bias, activation.  For few output channels per group
-// (the matrix kernel would multiply mostly padding) and for geometries past
-// its 16- and 32-bit offsets or its grid.
+// or small planes (the matrix kernels would multiply mostly padding) and for
+// geometries past their 16- and 32-bit offsets or their grid.
 __global__ __launch_bounds__(256) void k_conv2d_f32(const float *__restrict__ x, const float *__restrict__ w,
                                                     const float *__restrict__ bias, float *__restrict__ y, int C,
                                                     int H, int W, int Cout, int KH, int KW, int sh, int sw, int ph,
@@ -703,11 +704,64 @@ __global__ __launch_bounds__(256, 3) void k_conv2d_f32_patch(ConvF32 a) {
     }
 }
 
+// How many taps of one axis lie inside the image: the mean over its outputs
+// and how many do for any of them.
+struct LiveTaps {
+    double mean;
+    int any;
+};
+LiveTaps live_taps(int taps, int dil, int pad, int stride, int in, int out) {
+    LiveTaps l{0.0, 0};
+    for (int k = 0; k < taps; ++k) {
+        const int64_t at = (int64_t)k * dil - pad;  // input of output 0
+        const int64_t lo = at >= 0 ? 0 : (-at + stride - 1) / stride;
+        const int64_t hi = at >= in ? -1 : std::min<int64_t>(out - 1, (in - 1 - at) / stride);
+        if (hi < lo) continue;
+        l.mean += (double)(hi - lo + 1) / out;
+        ++l.any;
+    }
+    return l;
+}
+
+// Modelled times (us) of the three kernels, for the choice between the direct
+// one, which starts at once, wastes no lane on a plane's edge and skips the
+// taps in the padding, and the matrix kernels, whose workgroups compute 64 *
+// pb pixels of one image whatever its size.  Fitted to 1083 geometries (planes
+// of 1 to 112^2 pixels, 1 to 128 input and 4 to 256 output channels of a
+// group, 1 to 65536 images), the choice is the faster kernel or within 5 % of it on
+// 1030 of them, at most 27 % behind the direct and 65 % behind a matrix kernel.
+// 8 channels of 1x1x8 on 65536 single pixels: 6.7 us direct, 209 us matrix; 64
+// of 3x3x64 on 2048 planes of 4x4: 348 and 253 us.
+// The direct kernel: a chain of `live` products at cache latency, or all
+// chains at a rate that grows with the plane, since the lanes along a small
+// one read different channels' weights.
+double conv_direct_us(int64_t total, int64_t OHW, double live, bool one_tap) {
+    const double rate = 0.38e6 + 2.0e6 * std::min(1.0, (double)(OHW - 1) / 18.0);
+    return 2.2 + std::max(live * (one_tap ? 0.1 : 0.115), (double)total * live / rate) + (double)total / 2.27e5;
+}
+// The matrix kernels: what the first workgroup takes apart from its chains,
+// and per 256 workgroups; then the chains over K, in rounds of `resident`
+// workgroups per CU, and of the patch kernel (three per CU) the patch's
+// loads, in batches of 16 rows of 64 columns by each wavefront.
+double conv_matrix_us(bool patch, int64_t K, int64_t batches, int64_t workgroups, int cb, int pb) {
+    struct Fit {
+        double start, per_256, per_k, resident, per_batch;
+    };
+    constexpr Fit gather_fit[2][3] = {{{3.6, 0.45, 0.031, 2.0, 0}, {3.4, 0.46, 0.0434, 1.2, 0}, {3.65, 1.1, 0.065, 1.07, 0}},
+                                      {{3.5, 0.74, 0.059, 3.7, 0}, {5.2, 0.54, 0.083, 3.1, 0}, {15.8, 1.04, 0.0714, 1.34, 0}}};
+    constexpr Fit patch_fit[2][2] = {{{4.0, 1.4, 0.0144, 3.0, 2.27}, {5.1, 1.9, 0.0243, 3.0, 2.2}},
+                                     {{7.3, 0.76, 0.037, 3.0, 2.5}, {7.75, 2.2, 0.071, 3.0, 3.0}}};
+    const Fit &f = patch ? patch_fit[pb - 1][cb == 2 ? 0 : 1] : gather_fit[pb - 1][cb == 1 ? 0 : cb == 2 ? 1 : 2];
+    const double w = (double)workgroups / 256.0;
+    return f.start + f.per_256 * w + std::max(1.0, w / f.resident) * ((double)K * f.per_k + (double)batches * f.per_batch);
+}
+
 }  // namespace
 
 hipError_t launch_conv2d_f32(const float *x, const float *w, const float *bias, float *y, int64_t Nb, int C, int H,
                              int W, int Cout, int KH, int KW, int sh, int sw, int ph, int pw, int dh, int dw,
-                             int group, int OH, int OW, int act, hipStream_t s) {
+                             int group, int OH, int OW, int act, hipStream_t s, const char **kernel) {
+    *kernel = "conv2d_f32_direct";
     const int64_t total = Nb * Cout * OH * OW;
     if (total == 0) return hipSuccess;
     const int mg = Cout / group;
@@ -749,7 +803,15 @@ hipError_t launch_conv2d_f32(const float *x, const float *w, const float *bias, 
         if (patch_lds(pb) > kLdsMax) pb = 1;
         const bool patch = cb > 1 && K <= KT && patch_lds(pb) <= kLdsMax;
         if (!patch) pb = tiling(false, 2) * group * tiles_c >= 512 ? 2 : 1;
-        if (tiling(patch, pb) * group * tiles_c <= kGridMax) {
+        const int64_t workgroups = tiling(patch, pb) * group * tiles_c;
+        const LiveTaps lh = live_taps(KH, dh, ph, sh, H, OH), lw = live_taps(KW, dw, pw, sw, W, OW);
+        // (lanes of a wavefront wait for each other's taps: between the mean and the union)
+        const double k_live = (double)cg * std::sqrt(lh.mean * lw.mean * lh.any * lw.any);
+        const int64_t batches = (cg * ((4 * pb - 1) * (int64_t)sh + (KH - 1) * (int64_t)dh + 1) + 63) / 64 *
+                                ((15 * (int64_t)sw + (KW - 1) * (int64_t)dw + 64) / 64);
+        if (workgroups <= kGridMax && conv_matrix_us(patch, K, batches, workgroups, cb, pb) <=
+                                          conv_direct_us(total, OHW, k_live, KH * KW == 1)) {
+            *kernel = patch ? "conv2d_f32_patch" : "conv2d_f32_mfma";
             const int64_t lds = patch ? patch_lds(pb) : 0;
             const int64_t grid = group * tiles_c * (patch ? std::min<int64_t>(a.tiles, walk(lds)) : a.tiles);
             auto go = [&](auto cbv, auto pbv) -> hipError_t {

@@ -97,7 +97,7 @@ hipError_t launch_sgemm(int64_t M, int64_t N, int64_t K, const float *A, int64_t
                         int64_t ldb, int transB, const Epilogue &e, hipStream_t s);
 hipError_t launch_conv2d_f32(const float *x, const float *w, const float *bias, float *y, int64_t Nb, int C, int H,
                              int W, int Cout, int KH, int KW, int sh, int sw, int ph, int pw, int dh, int dw,
-                             int group, int OH, int OW, int act, hipStream_t s);
+                             int group, int OH, int OW, int act, hipStream_t s, const char **kernel);
 hipError_t launch_activation(const float *x, float *y, int64_t n, int act, hipStream_t s);
 
 // element formats of the fp8 data-type kernels (the ONNX type numbers)

@@ -124,3 +124,23 @@ def test_conv_f32_more_outputs_than_a_grid(dev):
     assert y.numel() > 1 << 32 and not bool(torch.isnan(y.view(-1)[-1000:]).any())
     for at in (slice(0, 999), slice((1 << 32) // cout - 500, (1 << 32) // cout + 7), slice(n - 500, n)):
         assert np.array_equal(y[at].cpu().numpy(), oracle.conv2d(x[at].cpu().numpy(), wt, np.zeros(cout, np.float32), group=3))
+
+
+# the choice of the kernel: small planes, single pixels, taps that mostly lie
+# in the padding and few products go to the direct kernel, the rest by their
+# channels and K to the other two
+@pytest.mark.parametrize("case,kernel", [((512, 16, 1, 1, 24, 1, 1, 1, 0, 1, 1), "direct"), ((300, 8, 4, 4, 9, 1, 1, 1, 0, 1, 1), "direct"),
+                                         ((40, 20, 1, 1, 20, 7, 7, 1, 3, 1, 1), "direct"), ((200, 12, 2, 2, 40, 3, 3, 1, 1, 1, 2), "direct"),
+                                         ((2, 30, 10, 10, 48, 1, 1, 1, 0, 1, 2), "direct"), ((3, 2, 30, 30, 3, 3, 3, 1, 1, 1, 1), "direct"),
+                                         ((4, 3, 57, 58, 40, 3, 3, 1, 1, 1, 1), "patch"), ((2, 24, 20, 21, 12, 3, 3, 1, 1, 1, 1), "mfma"),
+                                         ((1, 60, 4, 4, 70, 5, 5, 1, 2, 1, 1), "mfma")])
+def test_conv_f32_kernel(dev, case, kernel):
+    n, c, h, w, cout, kh, kw, st, pd, dl, group = case
+    x, b = synth.normal(c + h, (n, c, h, w)), synth.normal(3, (cout,), std=0.1)
+    wt = synth.normal(cout + kh, (cout, c // group, kh, kw), std=0.2)
+    capi.kernel_trace()
+    y = capi.conv2d_f32(torch.from_numpy(x).to(dev), torch.from_numpy(wt).to(dev), torch.from_numpy(b).to(dev),
+                        (st, st), (pd, pd), (dl, dl), group, act=capi.ACT_RELU)
+    assert capi.kernel_trace() == ["conv2d_f32_" + kernel]
+    ref = oracle.conv2d(x, wt, b, strides=(st, st), pads=(pd, pd), dilations=(dl, dl), group=group, act=oracle.ACT_RELU)
+    assert np.array_equal(y.cpu().numpy(), ref)
