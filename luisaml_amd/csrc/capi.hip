@@ -694,7 +694,9 @@ int lcml_fp8_sgemm(int64_t M, int64_t N, int64_t K, const float *a, int64_t lda,
     if (!a || !b) return fail(LCML_ERR_INVALID_ARG, "%s: NULL operand", fn);
     if (lda < (trans_a ? M : K) || ldb < (trans_b ? K : N))
         return fail(LCML_ERR_INVALID_ARG, "%s: leading dimension too small", fn);
-    return hip_status(lcml::launch_sgemm(M, N, K, a, lda, trans_a, b, ldb, trans_b, e, (hipStream_t)stream), fn);
+    const char *label = nullptr;
+    const hipError_t err = lcml::launch_sgemm(M, N, K, a, lda, trans_a, b, ldb, trans_b, e, (hipStream_t)stream, &label);
+    return hip_status(err, fn, label);
 }
 
 int lcml_fp8_activation(const float *x, float *y, int64_t n, int act, void *stream) {

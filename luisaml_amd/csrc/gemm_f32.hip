@@ -192,7 +192,7 @@ __global__ __launch_bounds__(256) void k_sgemm(int M, int N, int K, const float 
             }
 }
 
-// The general Gemm: any pitch and extent.  64x64 output tile per 256-thread
+// The general Gemm: any pitch and extent, and few k.  64x64 output tile per 256-thread
 // workgroup, 4x4 outputs per thread, one fma chain each, K staged through
 // LDS 16 at a time.
 constexpr int TM = 64, TN = 64, TK = 16;
@@ -860,7 +860,8 @@ void launch_sgemm_tile(int M, int N, int K, const float *A, int lda, bool a_kc, 
 }  // namespace
 
 hipError_t launch_sgemm(int64_t M, int64_t N, int64_t K, const float *A, int64_t lda, int transA, const float *B,
-                        int64_t ldb, int transB, const Epilogue &e, hipStream_t s) {
+                        int64_t ldb, int transB, const Epilogue &e, hipStream_t s, const char **kernel) {
+    *kernel = "lcml_fp8_sgemm_any";
     auto tiles = [&](int64_t t) { return ((M + t - 1) / t) * ((N + t - 1) / t); };
     // The tile, in units of one 16x16 block's chain (32 cycles per four
     // k): a workgroup of 64x64 runs four per SIMD, one of 32x32 one, but
@@ -868,10 +869,17 @@ hipError_t launch_sgemm(int64_t M, int64_t N, int64_t K, const float *A, int64_t
     const int64_t t64 = tiles(64), t32 = tiles(32), t16 = tiles(16);
     const double c64 = 4.0 * (double)((t64 + 255) / 256), c32 = std::max(1.25, 1.5 * (double)((t32 + 255) / 256));
     const int tb = t16 <= 256 ? 16 : c32 < c64 ? 32 : 64;
+    // Few k: the tiles' chunks of 32 to 128 are mostly padding, and three of
+    // them are loaded ahead.  M x N x K = 697 x 978 x 1: 4.8 us in general, 5.9
+    // by tiles; 59 x 1 x 1: 3.2 and 4.2; 762 x 73 x 6: 4.9 and 4.3, 254 x 33 x 7
+    // 4.9 and 4.3.  With many outputs up to K = 10: 3719 x 2932 x 7 23.0 and 27.9,
+    // 2812 x 426 x 9 6.5 and 8.9; 3136 x 1455 x 13 15.1 and 14.1.
+    const bool few_k = K <= 6 || (K <= 10 && M * N >= ((int64_t)1 << 19));
     // a tile's loads stay within 32-bit buffer extents: 128 rows of pitch
     constexpr int64_t kPitchMax = (int64_t)1 << 22;
-    if (lda < kPitchMax && ldb < kPitchMax && M < ((int64_t)1 << 30) && N < ((int64_t)1 << 30) &&
+    if (!few_k && lda < kPitchMax && ldb < kPitchMax && M < ((int64_t)1 << 30) && N < ((int64_t)1 << 30) &&
         K < ((int64_t)1 << 30) && tiles(tb) <= kGridMax) {
+        *kernel = "lcml_fp8_sgemm";
         // 16-byte loads: pointer, pitch and the extent they run along (K, or
         // the operand's rows) whole vectors
         auto whole = [](const float *p, int64_t ld, int64_t extent) {

@@ -58,6 +58,19 @@ def test_sgemm_infinities_stay_in_their_row(dev, tb):
     assert np.array_equal(sgemm(dev, a, b, 0, tb, bias, 0, 0), ref, equal_nan=True)
 
 
+# few k, also with many outputs, take the general kernel; either side of the lines
+@pytest.mark.parametrize("M,N,K,general", [(1, 1, 1, True), (59, 1, 1, True), (70, 130, 6, True), (70, 130, 7, False),
+                                           (723, 725, 7, False), (725, 724, 10, True), (725, 724, 11, False)])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_sgemm_few_k(dev, M, N, K, general, ta, tb):
+    a, b = synth.normal(M + K, (K, M) if ta else (M, K)), synth.normal(N + K, (N, K) if tb else (K, N))
+    bias = synth.normal(3, (N,))
+    capi.kernel_trace()
+    y = sgemm(dev, a, b, ta, tb, bias, 0, 0)
+    assert capi.kernel_trace() == ["lcml_fp8_sgemm_any" if general else "lcml_fp8_sgemm"]
+    assert np.array_equal(y, oracle.gemm(a, b, bias, transA=ta, transB=tb, act=oracle.ACT_RELU))
+
+
 def test_sgemm_more_tiles_than_a_grid(dev):
     """One row by 2^29 columns: more tiles than one grid dimension has workgroups."""
     N, K = (1 << 29) + 5, 25
