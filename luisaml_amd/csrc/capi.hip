@@ -653,10 +653,11 @@ int lcml_fp8_gemm_w8a32(int64_t M, int64_t N, int64_t K, const float *a, int64_t
     if (!a || !b_packed) return fail(LCML_ERR_INVALID_ARG, "%s: NULL operand", fn);
     if (lda < K || !aligned(a, 4)) return fail(LCML_ERR_INVALID_ARG, "%s: lda < K or a misaligned", fn);
     if (!aligned(b_packed, 16)) return fail(LCML_ERR_INVALID_ARG, "%s: b_packed not 16-byte aligned", fn);
-    return hip_status(lcml::w8a32_mfma_wins(M, N, K, lda)
-                          ? lcml::launch_gemm_w8a32(M, N, K, a, lda, b_packed, e, (hipStream_t)stream)
-                          : lcml::launch_gemv_valu_f32(M, N, K, a, lda, b_packed, e, (hipStream_t)stream),
-                      fn);
+    if (lcml::w8a32_mfma_wins(M, N, K, a, lda))
+        return hip_status(lcml::launch_gemm_w8a32(M, N, K, a, lda, b_packed, e, (hipStream_t)stream), fn,
+                          "gemm_w8a32_mfma");
+    return hip_status(lcml::launch_gemv_valu_f32(M, N, K, a, lda, b_packed, e, (hipStream_t)stream), fn,
+                      "gemv_valu_w8a32");
 }
 
 int lcml_fp8_conv2d_f32(const float *x, const float *w, const float *bias, float *y, int64_t n, int64_t c, int64_t h,

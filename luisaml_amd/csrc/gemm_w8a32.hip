@@ -279,19 +279,31 @@ Shape w8a32_shape(int64_t M, int64_t panels) {
     return c3 <= c2 && c3 <= c1 ? k32x3 : c2 < c1 ? k16x2 : k16x1;
 }
 
+bool w8a32_vec(const float *a, int64_t lda, int64_t K) {
+    return (reinterpret_cast<uintptr_t>(a) & 15) == 0 && lda % 4 == 0 && K % 4 == 0;
+}
+
 }  // namespace
 
 // Against the vector-ALU kernel, which starts a workgroup per row and panel
-// and needs no barriers: it stays for few of them and little work in each.
-// N = 256, K = 784: 3.4 us against 5.9 at M = 64, 5.3 at 128, 8.7 at 200;
-// N = K = 4096: 7.5 us against 11.9 at M = 4, 13.9 against 12.0 at 8;
-// N = 11008, K = 4096: 8.2 us against 15 at M = 1, 17.3 against 15.1 at 2;
-// N = 128, K = 256: 4.4 against 5.0 at M = 512; N = K = 512: 5.8 against 5.0
-// at M = 128.
-bool w8a32_mfma_wins(int64_t M, int64_t N, int64_t K, int64_t lda) {
+// (per two or four rows from 512 and 1024 of them) and needs no barriers, in
+// us (vector ALU / matrix cores):
+//   * up to 512 workgroups it stays, whatever K: N = 212, K = 6722, M = 56
+//     11.0 / 30.9; N = 982, K = 4333, M = 30 11.3 / 21.3; N = 1495, K = 4501,
+//     M = 12 10.8 / 18.2.  Few rows of many panels read the weights rather than
+//     share them: N = 11008, K = 4096, M = 1 8.2 / 15, 2 17.3 / 15.1; N = 2888,
+//     K = 4628, M = 8 16.2 / 13.6; N = 2882, K = 3550, M = 9 12.8 / 13.5;
+//   * up to 1024 with little work: N = 1007, K = 730 (4-byte loads), M = 61
+//     6.9 / 7.8; N = 150, K = 764 (16-byte loads), M = 339 8.2 / 5.9; N = 21, K =
+//     2655, M = 812 18.2 / 15.4; N = 256, K = 784, M = 200 8.7 / 5.9;
+//   * up to 2048 with next to none: N = 2500, K = 16, M = 39 4.5 / 5.0; N = 152, K = 60, M =
+//     391 7.6 / 4.9.
+bool w8a32_mfma_wins(int64_t M, int64_t N, int64_t K, const float *a, int64_t lda) {
     const int64_t panels = pad_to(N, kPanelCols) / 64;
-    const double w = (double)panels * (double)M;
-    if (w <= 1024 && w * (double)K <= (w <= 512 ? 1.1e6 : 3e5)) return false;
+    const double w = (double)panels * (double)M, wk = w * (double)K;
+    if (w <= 512 && !(M <= 8 && w > 256 && wk > 1.1e6)) return false;
+    if (w <= 1024 && wk <= (w8a32_vec(a, lda, K) ? 3e5 : 7.5e5)) return false;
+    if (w <= 2048 && wk <= 3e4) return false;
     // a row group's activations, a panel, and the grid at 16 rows per
     // workgroup of 512: a launch of 2^32 work items or more runs with that
     // number modulo 2^32 and reports no error
@@ -302,7 +314,7 @@ bool w8a32_mfma_wins(int64_t M, int64_t N, int64_t K, int64_t lda) {
 hipError_t launch_gemm_w8a32(int64_t M, int64_t N, int64_t K, const float *a, int64_t lda, const uint8_t *bp,
                              const Epilogue &e, hipStream_t s) {
     const int64_t panels = pad_to(N, kPanelCols) / 64, Kp = pad_to(K, kPackK);
-    const bool vec = (reinterpret_cast<uintptr_t>(a) & 15) == 0 && lda % 4 == 0 && K % 4 == 0;
+    const bool vec = w8a32_vec(a, lda, K);
     auto go = [&](auto mbv, auto pv, auto ksv, auto v) -> hipError_t {
         constexpr int MB = decltype(mbv)::value, P = decltype(pv)::value, KS = decltype(ksv)::value;
         constexpr bool V = decltype(v)::value;

@@ -85,7 +85,7 @@ hipError_t launch_gemm_skinny_dynamic(int64_t M, int64_t N, int64_t K, const flo
                                       hipStream_t s);
 // fp32 activations on the bf16 matrix cores (three exact pieces each), for the
 // sizes where they are the faster ones and within 32-bit buffer extents
-bool w8a32_mfma_wins(int64_t M, int64_t N, int64_t K, int64_t lda);
+bool w8a32_mfma_wins(int64_t M, int64_t N, int64_t K, const float *a, int64_t lda);
 hipError_t launch_gemm_w8a32(int64_t M, int64_t N, int64_t K, const float *a, int64_t lda, const uint8_t *bp,
                              const Epilogue &e, hipStream_t s);
 hipError_t launch_gemv_valu_f32(int64_t M, int64_t N, int64_t K, const float *a, int64_t lda,

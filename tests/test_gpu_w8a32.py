@@ -13,14 +13,17 @@ from luisaml_amd import capi, synth
 pytestmark = pytest.mark.gpu
 
 
-def run(dev, a, qw, sw, bias, pad=0, shift=0, out_dtype=torch.float32):
+def run(dev, a, qw, sw, bias, pad=0, shift=0, out_dtype=torch.float32, mfma=True):
     M, K = a.shape
     buf = torch.zeros(shift + M * (K + pad), dtype=torch.float32, device=dev)
     va = buf[shift:].view(M, K + pad)[:, :K]
     va.copy_(torch.from_numpy(a))
     bp = capi.pack_weight(torch.from_numpy(qw).to(dev), True)
-    return capi.gemm_w8a32(va, bp, torch.from_numpy(sw).to(dev), qw.shape[0], K, c=torch.from_numpy(bias).to(dev),
-                           out_dtype=out_dtype)
+    capi.kernel_trace()
+    y = capi.gemm_w8a32(va, bp, torch.from_numpy(sw).to(dev), qw.shape[0], K, c=torch.from_numpy(bias).to(dev),
+                        out_dtype=out_dtype)
+    assert capi.kernel_trace() == ["gemm_w8a32_mfma" if mfma else "gemv_valu_w8a32"]
+    return y
 
 
 def weights(N, K, seed):
@@ -47,7 +50,7 @@ def test_w8a32_against_64_bits(dev, M, N, K, pad, shift):
     a = synth.normal(M, (M, K)) * np.exp(synth.normal(M + 1, (M, K), std=3.0)).astype(np.float32)
     qw, sw = weights(N, K, N)
     bias = synth.normal(3, (N,), std=0.01)
-    check(run(dev, a, qw, sw, bias, pad, shift).cpu().numpy(), a, qw, sw, bias)
+    check(run(dev, a, qw, sw, bias, pad, shift, mfma=M > 1).cpu().numpy(), a, qw, sw, bias)
 
 
 def check_unscaled(y, a, B):
@@ -118,3 +121,18 @@ def test_w8a32_more_row_groups_than_a_grid(dev):
     y = torch.full((M, 1), np.nan, device=dev)
     capi.gemm_w8a32(a, capi.pack_weight(torch.from_numpy(qw).to(dev), True), torch.from_numpy(sw).to(dev), 1, 1, out=y)
     assert torch.equal(y, a * float(oracle.e4m3_to_float(qw)[0, 0]) * 0.5)
+
+
+# the choice of the kernel: rows and panels up to 512 on the vector ALU but for
+# a few rows of many panels over a long K; up to 1024 with little work, whose
+# bound depends on the activations' alignment; and next to no work
+@pytest.mark.parametrize("M,N,K,mfma", [(56, 212, 6722, False), (30, 982, 4333, False), (9, 2900, 3550, False), (8, 2900, 4628, True),
+                                        (4, 4100, 7312, True), (1, 11008, 4096, False), (2, 11008, 4096, True),
+                                        (61, 1007, 730, False), (61, 1007, 732, True), (339, 170, 200, False), (39, 2500, 16, False),
+                                        (391, 152, 60, True), (16, 4096, 512, True)])
+def test_w8a32_kernel(dev, M, N, K, mfma):
+    a = synth.normal(M, (M, K))
+    qw, sw = weights(N, K, N)
+    bias = synth.normal(3, (N,), std=0.01)
+    y = run(dev, a, qw, sw, bias, mfma=mfma)
+    check(y.cpu().numpy(), a, qw, sw, bias)
