@@ -190,7 +190,7 @@ __global__ __launch_bounds__(kThreads) void k_quantize_axis(const float *__restr
     }
 }
 
-// Scalar path: any alignment and size.
+// Scalar path: any alignment and size, and small tensors with a scale per axis.
 template <bool FROM_AMAX>
 __global__ __launch_bounds__(kThreads) void k_quantize_scalar(const float *__restrict__ x,
                                                               uint8_t *__restrict__ y, int64_t n,
@@ -564,12 +564,34 @@ ColsPlan plan_cols(int64_t n4, int64_t axis_len) {
 
 }  // namespace
 
+// Small tensors take an element per thread: the four-at-a-time kernels need
+// their loads, places, scales and reciprocals one after another, 2.6 to 5.5 us
+// however few there are, where a launch of the scalar kernel takes 2.1 us, and
+// 64-bit divisions per element cost it 3 us a million from there.  The lines are
+// where the two meet (quantize / dequantize, us, scalar and four at a time):
+//   * a scale per last-axis element: 524288 elements 3.0 and 3.1, 786432 3.5 and
+//     3.5 (dequantize: 2.1 and 2.1 from the smallest on);
+//   * runs that are not whole vectors, 63 long: 1.6 million 5.3 and 5.9, 2.1
+//     million 6.4 and 6.0 / 1.3 million 4.0 and 4.3, 2.1 million 5.3 and 4.7; 1023
+//     long, whose groups seldom cross into another scale: 1 million 4.1 and 4.2 /
+//     3.5 and 3.3;
+//   * runs of whole vectors: none is small enough (a launch of 4096 elements 3.5
+//     and 2.5, with the divisions done once per vector).
+namespace {
+bool quantize_small(int64_t n, int64_t inner) {
+    return inner == 1 ? n < 5 << 17 : inner % 4 != 0 && n < (inner < 256 ? 1 << 21 : 1 << 20);
+}
+bool dequantize_small(int64_t n, int64_t inner) {
+    return inner != 1 && inner % 4 != 0 && n < (inner < 256 ? 3 << 19 : 1 << 20);
+}
+}  // namespace
+
 hipError_t launch_quantize(const float *x, uint8_t *y, int64_t outer, int64_t axis_len,
                            int64_t inner, const float *scale, hipStream_t s, const char **kernel) {
     *kernel = "quantize_vec";
     const int64_t n = outer * axis_len * inner;
     if (n == 0) return hipSuccess;
-    const bool vec = aligned16(x) && aligned4(y);
+    const bool vec = aligned16(x) && aligned4(y) && (axis_len == 1 || !quantize_small(n, inner));
     if (vec && axis_len == 1) {
         hipLaunchKernelGGL(k_quantize_vec<false>, dim3(grid_vec(n / 4, kU)), dim3(kThreads), 0, s, x, y, n, scale,
                            nullptr, 0, nullptr);
@@ -599,7 +621,7 @@ hipError_t launch_dequantize(const uint8_t *x, float *y, int64_t outer, int64_t 
     *kernel = "dequantize_vec";
     const int64_t n = outer * axis_len * inner;
     if (n == 0) return hipSuccess;
-    const bool vec = aligned4(x) && aligned16(y);
+    const bool vec = aligned4(x) && aligned16(y) && (axis_len == 1 || !dequantize_small(n, inner));
     if (vec && axis_len == 1) {
         hipLaunchKernelGGL(k_dequantize_vec, dim3(grid_vec(n / 4, kUd)), dim3(kThreads), 0, s, x, y, n, scale);
     } else if (vec && inner == 1 && axis_len < ((int64_t)1 << 30)) {

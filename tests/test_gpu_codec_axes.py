@@ -44,6 +44,29 @@ def test_per_axis(dev, shape, axis, shift):
     assert np.array_equal(back.cpu().numpy(), oracle.dequantize(ref, s, axis=axis), equal_nan=True)
 
 
+# the smallest tensors of the four-at-a-time kernels and the largest scalar
+# ones: last-axis lengths 0..3 mod 4, one row, short rows; runs of 2, 3, 5, 7,
+# just under and over 256 and longer, whole vectors, outer repeats
+@pytest.mark.parametrize("shape,axis,quant,dequant", [
+    ((656, 1000), 1, "cols", "cols"), ((655, 1002), 1, "cols", "cols"), ((656, 1001), 1, "cols", "cols"), ((1, 655363), 1, "cols", "cols"),
+    ((218455, 3), 1, "cols", "cols"), ((2, 327681), 1, "cols", "cols"), ((655, 1000), 1, "scalar", "cols"),
+    ((1048577, 2), 0, "axis", "axis"), ((699053, 3), 0, "axis", "axis"), ((699050, 3), 0, "scalar", "axis"), ((7, 42801, 7), 1, "axis", "axis"),
+    ((2, 3, 70001, 5), 2, "axis", "axis"), ((3, 2100, 255), 1, "scalar", "axis"), ((3, 2743, 255), 1, "axis", "axis"), ((3, 1361, 257), 1, "axis", "axis"),
+    ((3, 1360, 257), 1, "scalar", "scalar"), ((1026, 1023), 0, "axis", "axis"), ((5, 7, 12), 1, "axis", "axis")])
+def test_per_axis_kernel(dev, shape, axis, quant, dequant):
+    x = special(synth.normal(sum(shape), shape))
+    s = np.abs(synth.normal(axis + 1, (shape[axis],), std=0.05)) + np.float32(1e-4)
+    s[0] = 1e-25  # outside the reciprocal's range
+    ds = torch.from_numpy(s).to(dev)
+    capi.kernel_trace()
+    q = capi.quantize(torch.from_numpy(x).to(dev), ds, axis=axis)
+    back = capi.dequantize(q, ds, axis=axis)
+    assert capi.kernel_trace() == ["quantize_" + quant, "dequantize_" + dequant]
+    ref = oracle.quantize(x, s, axis=axis)
+    assert np.array_equal(q.cpu().numpy(), ref)
+    assert np.array_equal(back.cpu().numpy(), oracle.dequantize(ref, s, axis=axis), equal_nan=True)
+
+
 @pytest.mark.parametrize("shape", [(1 << 10, (1 << 12) + 1, 1 << 10), (1 << 16, (1 << 16) + 1, 1), (3, 21, 68191747)])
 def test_per_axis_beyond_32_bits(dev, shape):
     """2^32 elements and more, with an inner run and without, whole vectors and not."""
