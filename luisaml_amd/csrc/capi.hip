@@ -139,9 +139,10 @@ int lcml_fp8_quantize_dynamic(const float *x, uint8_t *y, int64_t n, float *scal
         return fail(LCML_ERR_INVALID_ARG,
                     "lcml_fp8_quantize_dynamic: n=%lld needs a workspace of %d bytes", (long long)n,
                     LCML_FP8_DYNAMIC_WORKSPACE_BYTES);
-    return hip_status(lcml::launch_quantize_dynamic(x, y, n, scale_out, static_cast<uint32_t *>(workspace),
-                                                    (hipStream_t)stream),
-                      "lcml_fp8_quantize_dynamic");
+    const char *label = nullptr;
+    const hipError_t err = lcml::launch_quantize_dynamic(x, y, n, scale_out, static_cast<uint32_t *>(workspace),
+                                                         (hipStream_t)stream, &label);
+    return hip_status(err, "lcml_fp8_quantize_dynamic", label);
 }
 
 int lcml_fp8_amax(const float *x, int64_t n, float *amax_out, void *stream) {

@@ -28,7 +28,7 @@ int amax_partials_count(int64_t n);
 hipError_t launch_quantize_dynamic_parts(const float *x, uint8_t *y, int64_t n, const uint32_t *part, int npart,
                                          float *scale_out, hipStream_t s);
 hipError_t launch_quantize_dynamic(const float *x, uint8_t *y, int64_t n, float *scale_out,
-                                   uint32_t *work, hipStream_t s);
+                                   uint32_t *work, hipStream_t s, const char **kernel = nullptr);
 hipError_t launch_amax_to_float(const uint32_t *amax_bits, float *out, hipStream_t s);
 hipError_t launch_fill_u32(uint32_t *p, uint32_t v, int64_t n, hipStream_t s);
 

@@ -88,7 +88,7 @@ def test_per_axis_beyond_32_bits(dev, shape):
     assert capi.kernel_trace() == ["quantize_" + kind, "dequantize_" + kind]
 
 
-@pytest.mark.parametrize("n", [1, 3, 4, 5, 4097, 16387, 65533, 65537, 262147, 2097155, 9000001])
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 4097, 5003, 16387, 65533, 65537, 262147, 2097155, 9000001])
 @pytest.mark.parametrize("shift", [0, 1])
 def test_dynamic_odd_sizes(dev, n, shift):
     """The largest magnitude in the last element, so the tail sets the scale."""
@@ -102,6 +102,18 @@ def test_dynamic_odd_sizes(dev, n, shift):
     assert np.array_equal(q.cpu().numpy(), oracle.quantize(x, ref))
     back = capi.dequantize(q, s)
     assert np.array_equal(back.cpu().numpy(), oracle.dequantize(oracle.quantize(x, ref), ref))
+
+
+@pytest.mark.parametrize("n,kernel", [(1, "_small"), (255, "_small"), (4097, "_small"), (4999, "_small"), (5001, "_spread"), (4, "_spread"),
+                                      (4996, "_spread"), (65535, "_spread"), (65537, "")])
+def test_dynamic_kernel(dev, n, kernel):
+    x = synth.normal(n, (n,))
+    x[-1] = -9.0
+    capi.kernel_trace()
+    q, s = capi.quantize_dynamic(torch.from_numpy(x).to(dev))
+    assert capi.kernel_trace() == ["quantize_dynamic" + kernel]
+    ref = oracle.dynamic_scale(x)
+    assert float(s.item()) == ref and np.array_equal(q.cpu().numpy(), oracle.quantize(x, ref))
 
 
 @pytest.mark.parametrize("N,K", [(1, 1), (3, 15), (65, 16), (64, 17), (130, 255), (70, 1001), (33, 128), (5, 4099)])
