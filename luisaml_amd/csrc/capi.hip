@@ -313,6 +313,8 @@ int gemm_core(const char *fn, int64_t M, int64_t N, int64_t K, const uint8_t *a,
             return fail(LCML_ERR_UNSUPPORTED, "%s: M=%lld N=%lld exceeds the skinny kernel's grid", fn, (long long)M,
                         (long long)N);
         err = lcml::launch_gemm_skinny(M, N, K, a, lda, b_packed, e, kernel == LCML_KERNEL_SKINNY, s);
+        if (M <= 16 && lcml::skinny_col_blocks(N, K, false) < 4)
+            label = kernel == LCML_KERNEL_SKINNY ? "gemm_skinny_part" : "gemm_skinny_part_fp8";
         break;
     case LCML_KERNEL_VALU: err = lcml::launch_gemv_valu_fp8(M, N, K, a, lda, b_packed, e, s); break;
     default: return fail(LCML_ERR_INVALID_ARG, "%s: unknown kernel %d", fn, kernel);

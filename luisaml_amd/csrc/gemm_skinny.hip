@@ -657,10 +657,14 @@ int skinny_row_blocks(int64_t M, int64_t N, int64_t K, double *cost) {
 // wavefront and the weights stream through more CUs.  N = 4096 (a quarter),
 // E4M3 in, whole panels -> now: K = 4096 M = 1 7.7 -> 5.5 us, M = 16
 // 8.9 -> 6.6; K = 11008 16.3 -> 9.7 and 19.7 -> 12.0; N = 6144 (half), K = 4096,
-// M = 1 9.2 -> 6.9.
-int skinny_col_blocks(int64_t N) {
+// M = 1 9.2 -> 6.9.  A quarter's loads of four K blocks fetch nothing more for a
+// wavefront with one or two: E4M3 in, whole panels stay up to K = 2048 (N =
+// 4096, K = 1024, M = 1 3.3 us against 3.9 in quarters, K = 1536, N = 64, M = 16 3.8
+// against 4.1; K = 2560 4.5 against 4.5).  The fused quantiser encodes while the
+// loads run and gains from quarters at every K (K = 1024 4.9 -> 4.0).
+int skinny_col_blocks(int64_t N, int64_t K, bool fused) {
     const int64_t panels = (N + 63) / 64;
-    return panels > 128 ? 4 : panels > 64 ? 2 : 1;
+    return panels > 128 ? 4 : panels > 64 ? 2 : fused || K > 2048 ? 1 : 4;
 }
 
 hipError_t launch_gemm_skinny(int64_t M, int64_t N, int64_t K, const uint8_t *a, int64_t lda,
@@ -680,7 +684,7 @@ hipError_t launch_gemm_skinny(int64_t M, int64_t N, int64_t K, const uint8_t *a,
     // row blocks of 16 per workgroup (every weight fragment feeds MB MFMAs),
     // and row groups of 16*MB rows beyond that
     const int mb = skinny_row_blocks(M, N, K, nullptr);
-    const int nb = mb == 1 ? skinny_col_blocks(N) : NB;
+    const int nb = mb == 1 ? skinny_col_blocks(N, K, false) : NB;
     g.rg = (int)((M + 16 * mb - 1) / (16 * mb));
     const unsigned grid = (unsigned)(((N + 15) / 16 + nb - 1) / nb * g.rg);
 #define LCML_SKINNY_LAUNCH(NBV, MBV, UV)                                                                         \
@@ -723,7 +727,7 @@ hipError_t launch_gemm_skinny_dynamic(int64_t M, int64_t N, int64_t K, const flo
     g.rg = 1;
     g.e = e;
     constexpr int NB = LCML_SKINNY_NB, W = LCML_SKINNY_WAVES, U = LCML_SKINNY_UNROLL;
-    const int nb = skinny_col_blocks(N);
+    const int nb = skinny_col_blocks(N, K, true);
     const unsigned grid = (unsigned)(((N + 15) / 16 + nb - 1) / nb);
     const unsigned lds = (unsigned)skinny_dynamic_lds_bytes(M, K);
     // activation slots per lane per K block: ceil(M/2), rounded up to 1, 2,

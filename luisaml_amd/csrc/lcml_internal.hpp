@@ -68,6 +68,8 @@ hipError_t launch_gemm_skinny(int64_t M, int64_t N, int64_t K, const uint8_t *a,
 // the skinny kernel's 16-row blocks per workgroup (1, 2 or 4) for an M x N
 // output over K, and its modelled time in units of one 4-block workgroup's run
 int skinny_row_blocks(int64_t M, int64_t N, int64_t K, double *cost);
+// its 16-column blocks per workgroup (4 is a whole panel) for M <= 16
+int skinny_col_blocks(int64_t N, int64_t K, bool fused);
 // medium M behind a dynamic quantisation (exact): codes in 16-row blocks
 // (M*K bytes), then the GEMM that reads them, and its modelled time in us (1e30
 // for sizes it does not take)

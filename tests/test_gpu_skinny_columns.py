@@ -44,3 +44,17 @@ def test_columns_agree(dev, M, K, kernel):
         s = oracle.dynamic_scale(x)
         ref, A, B = oracle.qlinear(oracle.quantize(x, s), s, qw, sw, bias=bias, act=oracle.ACT_RELU)
         assert_close(full["gemm"], ref, oracle.gemm_abs_bound(A, B, bias))
+
+
+@pytest.mark.parametrize("N,K,part", [(64, 1024, False), (4096, 2048, False), (4096, 2064, True), (4097, 16, True), (8192, 1024, True),
+                                      (8193, 4096, False)])
+@pytest.mark.parametrize("M", [1, 16])
+def test_part_panels(dev, M, N, K, part):
+    """Quarters of a panel for a long K only, halves for 65 to 128 panels."""
+    a = torch.zeros((M, K), dtype=torch.uint8, device=dev)
+    bp = torch.zeros(capi.packed_weight_bytes(K, N), dtype=torch.uint8, device=dev)
+    one = torch.ones(1, device=dev)
+    capi.kernel_trace()
+    y = capi.gemm(a, one, bp, one, N, K)
+    assert capi.kernel_trace() == ["gemm_skinny_part" if part else "gemm_skinny"]
+    assert bool((y == 0).all())
