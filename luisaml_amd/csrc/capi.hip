@@ -239,11 +239,17 @@ int auto_gemm_kernel(int64_t M, int64_t N, int64_t K) { return auto_gemm_choice(
 // sum K in one chain, and a linear in one call equals its two calls), and its
 // modelled time is a seventh below (19 us a unit at K = 4096, 3 us besides).
 // N = 12288, K = 4096, with the quantiser: M = 100 31.7 us row-major against
-// 28.1.
-bool dynamic_by_rows(int64_t M, int64_t N, int64_t K) {
+// 28.1.  Up to 65536 elements of x the row-major codes take one launch where
+// these take two (unless x's partial maxima are given): 0.6 us on the
+// modelled times (N = 8192, K = 512, M = 32 8.9 us row-major against 9.9).
+// Up to 32 rows of 128 panels or more take 32 x 64 tiles and need a long K, in us
+// with the quantisers, row-major / these: N = 8192, M = 17 K = 2048 11.3 / 12.0,
+// 3072 13.0 / 13.2, 4096 16.4 / 14.9; N = 9216 11.3 / 12.0, 13.7 / 14.1, 16.6 / 14.9.
+bool dynamic_by_rows(int64_t M, int64_t N, int64_t K, bool x_parts) {
     const AutoChoice c = auto_gemm_choice(M, N, K);
-    return M > 16 && c.kernel == LCML_KERNEL_SKINNY &&
-           lcml::gemm_rows_us(M, N, K) < 0.86 * (c.units * 19.0 * (double)K / 4096.0 + 3.0);
+    const double launch = M * K <= LCML_FP8_DYNAMIC_SMALL_MAX && !x_parts ? 0.6 : 0.0;
+    return M > 16 && c.kernel == LCML_KERNEL_SKINNY && !(M <= 32 && N > 127 * 64 && K < 3584) &&
+           lcml::gemm_rows_us(M, N, K) + launch < 0.86 * (c.units * 19.0 * (double)K / 4096.0 + 3.0);
 }
 }  // namespace
 
@@ -428,7 +434,7 @@ int gemm_dynamic_impl(const char *fn, int64_t M, int64_t N, int64_t K, const flo
     uint8_t *q = ws;
     uint32_t *part = reinterpret_cast<uint32_t *>(ws + pad256(M * K));
     float *scale = x_scale_out ? x_scale_out : reinterpret_cast<float *>(ws + pad256(M * K) + LCML_FP8_DYNAMIC_WORKSPACE_BYTES);
-    if (kernel == LCML_KERNEL_AUTO && aligned(x, 16) && dynamic_by_rows(M, N, K)) {
+    if (kernel == LCML_KERNEL_AUTO && aligned(x, 16) && dynamic_by_rows(M, N, K, xa.part != nullptr)) {
         // medium M: the codes in the layout of the GEMM that reads them
         int npart = xa.npart;
         if (!xa.part)

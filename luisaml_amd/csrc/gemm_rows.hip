@@ -183,6 +183,8 @@ __global__ __launch_bounds__(kWaves * 64) void k_gemm_rows(const uint8_t *bp, co
 //   28 at 1536); 64 x 32: 6.5, at least 7 (10.8 at 256, 29 at 1024), and 32 x
 //   64 the same; 64 x 64, one per CU: 12 a round (15 at 256, 26 at 384, 39 at
 //   768); 96 x 64, one per CU: 17.3 a round (20 at 256, 55 at 768);
+// two 32 x 32 or wider share a CU, so past 256 of them whole rounds count (N = 1024,
+// K = 8192, M = 384, 384 of 32 x 32: 28.0 us row-major and 29.9, by 64 x 32 27.1);
 // 128 x 64 spills, 128 x 32 and 96 x 32 were slower than 64 x 32.  The weights
 // take N*K bytes at 4.3 TB/s at least.
 struct RowsShape {
@@ -196,7 +198,7 @@ RowsShape rows_shape(int64_t M, int64_t N, int64_t K) {
     RowsShape best{0, 0, 0.0};
     auto offer = [&](int mb, int nb, double slope, bool rounds, double least) {
         double w = (double)((rblocks + mb - 1) / mb * ((cblocks + nb - 1) / nb)) / 256.0;
-        if (rounds || (mb * nb >= 8 && w > 1.0)) w = (double)(int64_t)(w + 0.998);  // whole rounds
+        if (rounds || (mb * nb >= 4 && w > 1.0)) w = (double)(int64_t)(w + 0.998);  // whole rounds
         const double us = 3.0 + std::max({slope * w * kf, least * kf, memory});
         if (!best.mb || us < best.us) best = {mb, nb, us};
     };

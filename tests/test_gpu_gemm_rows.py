@@ -101,3 +101,16 @@ def test_one_call_equals_two(dev, M, N, K, out_dtype):
         codes, s = capi.quantize_dynamic(v)
         two = capi.gemm(codes, s, bp, sw, N, K, **kw)
         assert torch.equal(capi.gemm_dynamic(v, bp, sw, N, K, **kw), two)
+
+
+# either side of what the choice counts: the second launch for a small x, and a
+# short K under few rows of many panels
+@pytest.mark.parametrize("M,N,K,rows", [(32, 8192, 512, False), (65, 4096, 512, False), (100, 4096, 1024, True), (17, 8192, 3072, False),
+                                        (17, 8192, 4096, True), (32, 8128, 2048, True), (33, 8192, 2048, True), (200, 11008, 4096, False)])
+def test_rows_choice(dev, M, N, K, rows):
+    x = torch.ones((M, K), device=dev)
+    bp = torch.zeros(capi.packed_weight_bytes(K, N), dtype=torch.uint8, device=dev)
+    capi.kernel_trace()
+    y = capi.gemm_dynamic(x, bp, torch.ones(N, device=dev), N, K)
+    assert ("gemm_rows" in capi.kernel_trace()) == rows
+    assert bool((y == 0).all())
