@@ -341,21 +341,32 @@ __device__ __forceinline__ bool stage_weights(float *wl, __amdgpu_buffer_rsrc_t 
         lo[u] = k < k16 ? ((k >> 4) * 4 + (k & 3)) * WS + ((k >> 2) & 3) : -1;
     }
     constexpr int CU = NC / 4 < 8 ? NC / 4 : 8;  // channels loaded together
-    for (int ch = wave; ch < NC; ch += 4 * CU) {
-        float v[CU][KQ];
+    // 64 k at a time as many as there are (with the empty ones too 64 channels of
+    // 3x3x3 on 16 images of 56x56 take 19.7 us instead of 17.6)
+    auto channels = [&](auto nq) {
+        constexpr int Q = decltype(nq)::value;
+        for (int ch = wave; ch < NC; ch += 4 * CU) {
+            float v[CU][Q];
 #pragma unroll
-        for (int i = 0; i < CU; ++i)
+            for (int i = 0; i < CU; ++i)
 #pragma unroll
-            for (int u = 0; u < KQ; ++u)  // kOOB plus a channel's offset stays out of range
-                v[i][u] = buf_f32(wr, ch + 4 * i < nch ? wo[u] + (uint32_t)((ch + 4 * i) * K) * 4u : kOOB);
+                for (int u = 0; u < Q; ++u)  // kOOB plus a channel's offset stays out of range
+                    v[i][u] = buf_f32(wr, ch + 4 * i < nch ? wo[u] + (uint32_t)((ch + 4 * i) * K) * 4u : kOOB);
 #pragma unroll
-        for (int i = 0; i < CU; ++i)
+            for (int i = 0; i < CU; ++i)
 #pragma unroll
-            for (int u = 0; u < KQ; ++u) {
-                bad |= !(fabsf(v[i][u]) <= 3.4028235e38f);
-                if (lo[u] >= 0) wl[lo[u] + (ch + 4 * i) * 4] = v[i][u];
-            }
-    }
+                for (int u = 0; u < Q; ++u) {
+                    bad |= !(fabsf(v[i][u]) <= 3.4028235e38f);
+                    if (lo[u] >= 0) wl[lo[u] + (ch + 4 * i) * 4] = v[i][u];
+                }
+        }
+    };
+    if (k16 <= 64)
+        channels(std::integral_constant<int, 1>{});
+    else if (k16 <= 128)
+        channels(std::integral_constant<int, 2>{});
+    else
+        channels(std::integral_constant<int, KQ>{});
     return bad;
 }
 
@@ -517,27 +528,28 @@ __global__ __launch_bounds__(256) void k_conv2d_f32_mfma(ConvF32 a) {
     });
 }
 
-// The same chain with the input staged too, for K of one part: a workgroup
-// walks tiles of 16 output columns x 4*PB rows of one image (a wavefront PB
-// rows, a lane one column), and the input under a tile (all channels of the
-// group, zeros in the padding) lies in LDS, so that a pixel's value costs one
-// LDS read and one addition instead of a bounds test and a load, and the
+// The same chain with the input staged too, for K of one part (at most KT) and
+// more than 16 channels: a workgroup walks tiles of 16 output columns x 4*PB
+// rows of one image (a wavefront PB rows, a lane one column), and the input
+// under a tile (all channels of the group, zeros in the padding) lies in LDS,
+// so that a pixel's value costs one LDS read and one addition instead of a bounds test and a load, and the
 // weights are staged once per workgroup.  The LDS reads of the next 16 k's are
 // issued before the MFMAs of the current ones; three workgroups per CU
 // (at most 168 VGPRs) keep the matrix units busy while others stage: with two,
 // the tile's loads and stores left them idle half the time.  Stem of a
-// ResNet (64 channels of 7x7x3, stride 2, 16 images of 224x224): 62 us against
+// ResNet (64 channels of 7x7x3, stride 2, 16 images of 224x224): 55 us against
 // 76 us with the values gathered, 72 us with two workgroups per CU, 1010 us
 // one thread per output; 24 us at the full MFMA rate.
 template <int CB, int PB>
 __global__ __launch_bounds__(256, 3) void k_conv2d_f32_patch(ConvF32 a) {
+    static_assert(CB > 1, "16 channels or fewer: the gather kernel");
     constexpr int NC = CB * 16, WS = kWS<CB>;
     extern __shared__ __attribute__((aligned(16))) float smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int ct = (int)blockIdx.x % a.tiles_c, grp = (int)blockIdx.x / a.tiles_c % a.group;
     const int first = (int)blockIdx.x / (a.tiles_c * a.group), step = (int)gridDim.x / (a.tiles_c * a.group);
     const int cg = a.C / a.group, mg = a.Cout / a.group, taps = a.KH * a.KW, K = taps * cg;
-    const int HW = a.H * a.W, OHW = a.OH * a.OW, KP = (min(K, KT) + 15) / 16 * 16;
+    const int HW = a.H * a.W, OHW = a.OH * a.OW, KP = (K + 15) / 16 * 16;
     const int PH = (4 * PB - 1) * a.sh + (a.KH - 1) * a.dh + 1, PW = 15 * a.sw + (a.KW - 1) * a.dw + 1;
     float *wl = smem, *bias_l = smem + KP / 4 * WS + KP, *patch = bias_l + NC;
     int *tab = reinterpret_cast<int *>(smem + KP / 4 * WS);  // k's offset in the patch, at (k/16)*16 + (k%4)*4 + (k/4)%4
@@ -586,7 +598,7 @@ __global__ __launch_bounds__(256, 3) void k_conv2d_f32_patch(ConvF32 a) {
         for (int u = 0; u < RU; ++u)
             if (col < PW && row0 + 4 * u < nrow) patch[(row0 + 4 * u) * PW + col] = v[u];
     };
-    bool bad_any = false;
+    bool bad = false;
     for (int tile = first; tile < a.tiles; tile += step) {
         const Tile tl = place(tile);
         const int oh0 = tl.oh0, ow0 = tl.ow0, ih0 = tl.ih0, iw0 = tl.iw0, n = tl.n;
@@ -598,44 +610,39 @@ __global__ __launch_bounds__(256, 3) void k_conv2d_f32_patch(ConvF32 a) {
                 store_rows(r0, c0 + lane, v);
             }
         if (tile == first && tid < NC) bias_l[tid] = buf_f32(br, (uint32_t)tid * 4u);
+        if (tile == first) {  // the weights and the table, for all tiles
+            for (int k = tid; k < KP; k += 256) {
+                int t = 0;  // past K: any value, masked below
+                if (k < K) {
+                    const int tp = k / cg, c = k - tp * cg, kh = tp / a.KW, kw = tp - kh * a.KW;
+                    t = (c * PH + kh * a.dh) * PW + kw * a.dw;
+                }
+                tab[(k & ~15) + (k & 3) * 4 + ((k >> 2) & 3)] = t;
+            }
+            bad = __syncthreads_or(stage_weights<CB>(wl, wr, nch, 0, K, cg, taps, K));
+        } else {
+            __syncthreads();
+        }
         f4 acc[PB][CB] = {};
-        for (int kt = 0; kt < K; kt += KT) {
-            const int kn = min(KT, K - kt), ng = (kn + 15) / 16;
-            if (K > KT || tile == first) {  // one part: staged once for all tiles
-                if (kt) __syncthreads();    // the previous part is consumed
-                for (int k = tid; k < KP; k += 256) {
-                    int t = 0;  // past K: any value, masked below
-                    if (k < kn) {
-                        const int tp = (kt + k) / cg, c = kt + k - tp * cg, kh = tp / a.KW, kw = tp - kh * a.KW;
-                        t = (c * PH + kh * a.dh) * PW + kw * a.dw;
-                    }
-                    tab[(k & ~15) + (k & 3) * 4 + ((k >> 2) & 3)] = t;
+        if (__builtin_expect(bad, 0)) {
+            for (int k = 0; k < K; ++k) {
+                const int tp = k / cg, kh = tp / a.KW, kw = tp - kh * a.KW;
+                const int t = tab[(k & ~15) + (k & 3) * 4 + ((k >> 2) & 3)], iw = iw0 + (lane & 15) * a.sw + kw * a.dw;
+#pragma unroll
+                for (int i = 0; i < PB; ++i) {
+                    const int ih = ih0 + (pr + i) * a.sh + kh * a.dh;
+                    const float xv = patch[pb0 + i * pbs + t];
+                    if ((uint32_t)ih < (uint32_t)a.H && (uint32_t)iw < (uint32_t)a.W)
+#pragma unroll
+                        for (int c = 0; c < CB; ++c)
+#pragma unroll
+                            for (int r = 0; r < 4; ++r)
+                                acc[i][c][r] =
+                                    fmaf(xv, wl[((k >> 4) * 4 + (k & 3)) * WS + (c * 16 + chl + r) * 4 + ((k >> 2) & 3)],
+                                         acc[i][c][r]);
                 }
-                const bool bad = stage_weights<CB>(wl, wr, nch, kt, kn, cg, taps, K);
-                bad_any = __syncthreads_or(bad);
-            } else {
-                __syncthreads();
             }
-            if (bad_any) {
-                for (int k = 0; k < kn; ++k) {
-                    const int tp = (kt + k) / cg, kh = tp / a.KW, kw = tp - kh * a.KW;
-                    const int t = tab[(k & ~15) + (k & 3) * 4 + ((k >> 2) & 3)], iw = iw0 + (lane & 15) * a.sw + kw * a.dw;
-#pragma unroll
-                    for (int i = 0; i < PB; ++i) {
-                        const int ih = ih0 + (pr + i) * a.sh + kh * a.dh;
-                        const float xv = patch[pb0 + i * pbs + t];
-                        if ((uint32_t)ih < (uint32_t)a.H && (uint32_t)iw < (uint32_t)a.W)
-#pragma unroll
-                            for (int c = 0; c < CB; ++c)
-#pragma unroll
-                                for (int r = 0; r < 4; ++r)
-                                    acc[i][c][r] = fmaf(
-                                        xv, wl[((k >> 4) * 4 + (k & 3)) * WS + (c * 16 + chl + r) * 4 + ((k >> 2) & 3)],
-                                        acc[i][c][r]);
-                    }
-                }
-                continue;
-            }
+        } else {
             struct Frag {
                 float x[PB][4];
                 f4 w[CB];
@@ -658,7 +665,7 @@ __global__ __launch_bounds__(256, 3) void k_conv2d_f32_patch(ConvF32 a) {
                     for (int i = 0; i < PB; ++i)
                         acc[i][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.w[c][j], f.x[i][j], acc[i][c], 0, 0, 0);
             };
-            const int gl = ng - 1;  // the last group, which may be partial
+            const int gl = KP / 16 - 1;  // the last group, which may be partial
             Frag f0, f1;
             fetch(f0, 0, offs(0));
             i4 t = offs(min(1, gl));
@@ -682,9 +689,9 @@ __global__ __launch_bounds__(256, 3) void k_conv2d_f32_patch(ConvF32 a) {
             // k past K: its weights are zero, and its value has to be finite
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                if (gl * 16 + 4 * j >= kn) break;
+                if (gl * 16 + 4 * j >= K) break;
 #pragma unroll
-                for (int i = 0; i < PB; ++i) f0.x[i][j] = gl * 16 + 4 * j + q < kn ? f0.x[i][j] : 0.0f;
+                for (int i = 0; i < PB; ++i) f0.x[i][j] = gl * 16 + 4 * j + q < K ? f0.x[i][j] : 0.0f;
                 mma(f0, j);
             }
         }
@@ -816,16 +823,19 @@ hipError_t launch_conv2d_f32(const float *x, const float *w, const float *bias, 
             const int64_t grid = group * tiles_c * (patch ? std::min<int64_t>(a.tiles, walk(lds)) : a.tiles);
             auto go = [&](auto cbv, auto pbv) -> hipError_t {
                 constexpr int CB = decltype(cbv)::value, PB = decltype(pbv)::value;
-                if (patch) {
-                    static std::atomic<uint64_t> lds_set{0};
-                    if (hipError_t err = ensure_dynamic_lds(reinterpret_cast<const void *>(k_conv2d_f32_patch<CB, PB>),
-                                                            (int)kLdsMax, lds_set);
-                        err != hipSuccess)
-                        return err;
-                    hipLaunchKernelGGL((k_conv2d_f32_patch<CB, PB>), dim3((unsigned)grid), dim3(256), (unsigned)lds, s, a);
-                } else {
-                    hipLaunchKernelGGL((k_conv2d_f32_mfma<CB, PB>), dim3((unsigned)grid), dim3(256), 0, s, a);
+                if constexpr (CB > 1) {
+                    if (patch) {
+                        static std::atomic<uint64_t> lds_set{0};
+                        if (hipError_t err = ensure_dynamic_lds(
+                                reinterpret_cast<const void *>(k_conv2d_f32_patch<CB, PB>), (int)kLdsMax, lds_set);
+                            err != hipSuccess)
+                            return err;
+                        hipLaunchKernelGGL((k_conv2d_f32_patch<CB, PB>), dim3((unsigned)grid), dim3(256), (unsigned)lds,
+                                           s, a);
+                        return hipGetLastError();
+                    }
                 }
+                hipLaunchKernelGGL((k_conv2d_f32_mfma<CB, PB>), dim3((unsigned)grid), dim3(256), 0, s, a);
                 return hipGetLastError();
             };
             using One = std::integral_constant<int, 1>;
