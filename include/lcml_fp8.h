@@ -329,7 +329,9 @@ LCML_API int lcml_fp8_conv2d(const uint8_t *x_nhwc, const float *x_scale, int64_
  * This is the reference graph DequantizeLinear(W) -> Gemm with unquantised
  * activations (the 3-layer MLP).  A few rows and panels run the VALU kernel;
  * more run on the bf16 matrix cores, each activation as the exact sum of three
- * bf16 values, accumulated in fp32.
+ * bf16 values, accumulated in fp32.  The kernel and its split of K follow M and
+ * N, so a row's rounding may differ with the number of rows it is computed
+ * with (as lcml_fp8_gemm's with its kernel).
  */
 LCML_API int lcml_fp8_gemm_w8a32(int64_t M, int64_t N, int64_t K, const float *a, int64_t lda,
                         const uint8_t *b_packed, const float *b_scale, int b_scale_per_channel,

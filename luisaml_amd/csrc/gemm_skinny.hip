@@ -5,7 +5,8 @@
 // as 128-bit loads in packed-panel order (no LDS staging: every weight byte
 // is used by exactly one wavefront).  A workgroup of WAVES wavefronts owns
 // 16*NB output columns (NB = 4: one whole 64-column panel, so every k-chunk
-// row of 1 KB is read contiguously by one workgroup); the wavefronts split K,
+// row of 1 KB is read contiguously by one workgroup; NB = 2 or 1, half a panel
+// or a quarter, for few columns at M <= 16); the wavefronts split K,
 // each issues the weight loads of UNROLL K blocks before their MFMAs, and the
 // partial 16x16 tiles are summed through LDS before the epilogue.  The
 // activations (M <= 16 rows, padded to 16 with zeros) are re-read from L2 by
@@ -30,13 +31,15 @@
 // the same M*K floats) and derives the per-tensor scale amax/448 exactly as
 // the standalone dynamic quantiser does.  Each wavefront then encodes the
 // activations of its own K blocks into LDS (row pitch Kp+16 bytes, so the 16
-// rows of a fragment read fall in distinct banks; k >= K is zero), one block
-// at a time, right after issuing that block's weight loads: the ~40 VALU
-// operations per float4 of the exact encode run while the weights are in
-// flight, and only the first block's encode delays the stream.  When a
-// wavefront's blocks fit its 4 or 8 activation slots (ONE), the amax pass
-// already loads x in the per-block layout and the encode reuses those
-// registers, so x is read once.  (Encoding all of x before the main loop cost 1.55 us at
+// rows of a fragment read fall in distinct banks; k >= K is zero), with NB = 4
+// one block at a time, right after issuing that block's weight loads: the ~40
+// VALU operations per float4 of the exact encode run while the weights are in
+// flight, and only the first block's encode delays the stream.  With NB < 4 two
+// or four blocks of weights are in flight anyway, and all of a wavefront's
+// blocks are encoded before the first product.  When a wavefront's blocks fit
+// its 4 or 8 (NB < 4: or 16) activation slots (ONE), the amax pass already
+// loads x in the per-block layout and the encode reuses those registers, so x
+// is read once.  (Encoding all of x before the main loop cost 1.55 us at
 // M=1 and 2.6 us at M=4 over the E4M3-in kernel on the 4096x11008 linear;
 // per block with one read of x, 0.6 and 1.0 us.)  The redundant
 // per-workgroup amax and encode still cost M*K loads and VALU work in every
@@ -167,8 +170,9 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_skinny(const uint8_t *bp, c
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) a_ok[mb] = row0 + mb * 16 + arow < M;
 
-    // weights: this workgroup's 64-column panel (the grid covers the panels
-    // exactly, so its four 16-column blocks all exist).  Lane l reads column
+    // weights: this workgroup's NB 16-column blocks of one 64-column panel (the
+    // grid covers the columns in units of NB blocks, and a panel is packed
+    // whole, so they all exist).  Lane l reads column
     // l%16 of each block and half l/16 of each k-chunk: block j's two
     // 16-byte pieces of a K block lie at b_lane + j*256 and + 1024 from the
     // K block's first byte.
@@ -731,8 +735,9 @@ hipError_t launch_gemm_skinny_dynamic(int64_t M, int64_t N, int64_t K, const flo
     const unsigned grid = (unsigned)(((N + 15) / 16 + nb - 1) / nb);
     const unsigned lds = (unsigned)skinny_dynamic_lds_bytes(M, K);
     // activation slots per lane per K block: ceil(M/2), rounded up to 1, 2,
-    // 4, 8; one round of 4 or 8 activation loads when a wavefront's K blocks
-    // (at most ceil(nkb / W)) take at most that many slots
+    // 4, 8; one round of 4 or 8 (parts of a panel, M <= 4: or 16) activation
+    // loads when a wavefront's K blocks (at most ceil(nkb / W)) take at most
+    // that many slots
     auto run_nb = [&](auto nbv, auto uv, auto sb, auto one) -> hipError_t {
         constexpr int B = decltype(nbv)::value, UV = decltype(uv)::value;
         constexpr int SB = decltype(sb)::value;

@@ -4,22 +4,23 @@
 // Every E4M3 weight is a bf16 value, and every finite fp32 activation is the
 // sum of three: hi, its upper 16 bits; mid, the upper 16 bits of x - hi; and
 // lo, what is left (24 bits in three pieces of 8; both differences are
-// exact).  The nine bits of a product of pieces are exact in the matrix
-// unit, which accumulates in fp32, so hi, mid and lo through three
+// exact).  A piece times a weight, 8 bits by 4, is exact in the matrix unit,
+// which accumulates in fp32, so hi, mid and lo through three
 // v_mfma_f32_16x16x32_bf16 give sum_k x_k w_k with fewer roundings than an fma
 // chain over k has (one per 32 products; error against 64 bits at 128 x 11008
-// x 4096 1.1e-7 of the norm, 3.0e-7 with the fma chains).  Three of them take 48 cycles of a
-// SIMD for 8192 multiply-adds; v_fma_f32 takes 512.  The activations are
-// split times 2^16, so that bf16's smallest value, 2^-133, holds the last bit of
-// every one, subnormals among them, and the sums are scaled back.
+// x 4096 1.5e-7 of the norm, 3.3e-7 with the fma chains).  Three of them take
+// 48 cycles of a SIMD for 8192 multiply-adds; v_fma_f32 takes 512.  The
+// activations are split times 2^16, so that bf16's smallest value, 2^-133,
+// holds the last bit of every one, subnormals among them, and the sums are
+// scaled back.
 //
-// What is left is shaped as the small-M FP8 GEMM: a workgroup of 8
-// wavefronts owns 16*MB rows and one 64-column panel; the wavefronts split K
-// in blocks of 128, read weights and activations straight into registers
-// (each weight byte is used by one wavefront) one block ahead, and sum their
-// partial tiles through LDS.  Splitting an activation costs 5.5 VALU
-// operations and is repeated by every panel's workgroup; beside 12 MFMAs per
-// 16 of them it hides.
+// What is left is to feed them.  A workgroup owns 16*MB rows and P 64-column
+// panels and splits K in KS parts, one wavefront to a panel and part, that
+// sum their tiles through LDS at the end.  The weights go straight to
+// registers, each byte to one wavefront; the activations pass through LDS,
+// split once per workgroup (6.5 VALU operations each, beside 12 MFMAs per 16
+// of them per panel), 64 k a step.  The K split, and with it the order of a
+// row's sum, depends on M and N.
 //
 // An activation that is inf, NaN or from 2^112 on leaves NaN in mid and lo.
 // The wavefronts test their sums for NaN and infinities once, at the end, and
@@ -267,9 +268,9 @@ __global__ __launch_bounds__(P *KS * 64, P == 2 && VEC ? 4 : 1) void k_gemm_w8a3
 // The shapes: 16 rows x 1 panel with K in 8 parts, 16 x 2 in 4, 32 x 3 in 4.
 // A round of up to 256 workgroups (one per CU) takes 12.5, 15.5 and 34 us at
 // K = 4096, all in proportion to K, so the larger shapes win where the work
-// fills their rounds: N = 11008 at M = 16: 16 us (19, 30 with the other two),
-// M = 64: 29 us (40, 33), M = 128: 39 us (73, 47), M = 512: 145 us (274, 161).
-// Wider still (32 x 4 in 2): 48 us at M = 128, 141 us at M = 512.
+// fills their rounds: N = 11008 at M = 16: 15 us (19, 30 with the other two),
+// M = 64: 28 us (40, 33), M = 128: 35 us (73, 47), M = 512: 141 us (274, 161).
+// Wider still (32 x 4 in 2): 48 us at M = 128, the same at M = 512.
 enum Shape { k16x1, k16x2, k32x3 };
 Shape w8a32_shape(int64_t M, int64_t panels) {
     auto rounds = [&](int64_t rows, int64_t p) {
@@ -296,8 +297,8 @@ bool w8a32_vec(const float *a, int64_t lda, int64_t K) {
 //   * up to 1024 with little work: N = 1007, K = 730 (4-byte loads), M = 61
 //     6.9 / 7.8; N = 150, K = 764 (16-byte loads), M = 339 8.2 / 5.9; N = 21, K =
 //     2655, M = 812 18.2 / 15.4; N = 256, K = 784, M = 200 8.7 / 5.9;
-//   * up to 2048 with next to none: N = 2500, K = 16, M = 39 4.5 / 5.0; N = 152, K = 60, M =
-//     391 7.6 / 4.9.
+//   * up to 2048 with next to none: N = 2500, K = 16, M = 39 4.5 / 5.0; N = 152,
+//     K = 60, M = 391 7.6 / 4.9.
 bool w8a32_mfma_wins(int64_t M, int64_t N, int64_t K, const float *a, int64_t lda) {
     const int64_t panels = pad_to(N, kPanelCols) / 64;
     const double w = (double)panels * (double)M, wk = w * (double)K;
