@@ -532,9 +532,10 @@ __global__ __launch_bounds__(256) void k_conv2d_f32_mfma(ConvF32 a) {
 // more than 16 channels: a workgroup walks tiles of 16 output columns x 4*PB
 // rows of one image (a wavefront PB rows, a lane one column), and the input
 // under a tile (all channels of the group, zeros in the padding) lies in LDS,
-// so that a pixel's value costs one LDS read and one addition instead of a bounds test and a load, and the
-// weights are staged once per workgroup.  The LDS reads of the next 16 k's are
-// issued before the MFMAs of the current ones; three workgroups per CU
+// so that a pixel's value costs one LDS read and one addition instead of a
+// bounds test and a load, and the weights are staged once per workgroup.  The
+// LDS reads of the next 16 k's are issued before the MFMAs of the current
+// ones; three workgroups per CU
 // (at most 168 VGPRs) keep the matrix units busy while others stage: with two,
 // the tile's loads and stores left them idle half the time.  Stem of a
 // ResNet (64 channels of 7x7x3, stride 2, 16 images of 224x224): 55 us against
@@ -735,10 +736,11 @@ LiveTaps live_taps(int taps, int dil, int pad, int stride, int in, int out) {
 // taps in the padding, and the matrix kernels, whose workgroups compute 64 *
 // pb pixels of one image whatever its size.  Fitted to 1083 geometries (planes
 // of 1 to 112^2 pixels, 1 to 128 input and 4 to 256 output channels of a
-// group, 1 to 65536 images), the choice is the faster kernel or within 5 % of it on
-// 1030 of them, at most 27 % behind the direct and 65 % behind a matrix kernel.
-// 8 channels of 1x1x8 on 65536 single pixels: 6.7 us direct, 209 us matrix; 64
-// of 3x3x64 on 2048 planes of 4x4: 348 and 253 us.
+// group, 1 to 65536 images), the choice is the faster kernel or within 5 % of
+// it on 1030 of them, at most 27 % behind the direct and 65 % behind a matrix
+// kernel.  8 channels of 1x1x8 on 65536 single pixels: 6.7 us direct, 209 us
+// matrix; 64 of 3x3x64 on 2048 planes of 4x4: 348 and 253 us.
+//
 // The direct kernel: a chain of `live` products at cache latency, or all
 // chains at a rate that grows with the plane, since the lanes along a small
 // one read different channels' weights.
